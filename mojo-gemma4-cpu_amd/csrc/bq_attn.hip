@@ -14,23 +14,24 @@
 // (p & row_mask).  Q codes are [token][q_head][head_dim] int8 with
 // qi_bias = 128 * sum(codes) and f_q = amax per (token, q_head).
 //
-// Flash attention: one wave per (token, kv head, split).  The split is a
-// contiguous range of the token's KV positions (worker_range of the range
-// into S = min(s_max, ceil(L / kAttnMinSplit)) parts).  A wave walks its
-// range in tiles of 16 positions exactly as the reference does: the 16 x G
-// scores of a tile come from head_dim/64 int8 MFMAs (A = the G query heads
-// of this kv head, B = 16 K rows); per head the tile max, corr and weights
-// use the reference's fast exp and its 16-lane tree sum; then acc *= corr and
-// acc += (w * vs / 127) * v position by position, each lane owning head_dim/64
-// consecutive output columns of every head.  A token whose range is one split
-// of a sliding layer is finalized in the wave (acc * (1/l), the sliding
-// prefill kernel), and so is every token of a one-split plan (full layers:
-// the merge of one split); every other token's splits are written as
-// (m, l, acc) partials and merged by k_attn_merge / k_attn_merge_lds in split
-// order with the reference's merge (corrections masked by l > 0, a 16-lane
-// tree per batch of 16 splits, the first contributing split multiplied, the
-// rest fma-accumulated).  One-split plans with head_dim <= 256 run
-// k_flash_attn_mt instead: 16/G tokens per wave on a shared tile grid.
+// Flash attention.  A split is a contiguous range of a token's KV positions
+// (worker_range of the range into S = min(s_max, ceil(L / kAttnMinSplit))
+// parts), walked in tiles of 16 positions exactly as the reference does: the
+// scores of a tile come from head_dim/64 int8 MFMAs (A = 16 rows of query
+// heads, B = 16 K rows); per head the tile max, corr and weights use the
+// reference's fast exp and its 16-lane tree sum; then acc *= corr and acc +=
+// (w * vs / 127) * v position by position.  Two kernels:
+//   k_flash_attn       decode: one wave per (token, kv head, split)
+//   k_flash_attn_rows  prefill chunks: 16/G tokens share every K/V tile
+// A token whose range is one split of a sliding layer is finalized there
+// (acc * (1/l), the sliding prefill kernel), and so is every token of a
+// one-split plan (full layers: the merge of one split); every other token's
+// splits are written as (m, l, acc) partials and merged by k_attn_merge in
+// split order with the reference's merge (corrections masked by l > 0, a
+// 16-lane tree per batch of 16 splits, the first contributing split
+// multiplied, the rest fma-accumulated).
+#include <type_traits>
+
 #include "bq_kernels.hpp"
 #include "bq_device.hpp"
 
@@ -79,6 +80,14 @@ __device__ inline float max87(float x) { return x > -87.0f ? x : -87.0f; }
 
 __device__ inline float readlane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// workgroups of k_flash_attn_rows per group of 16 / G tokens: four tokens each
+// where it takes them one per wave
+__host__ __device__ constexpr int attn_rows_parts(int G) { return G <= 2 ? 4 / G : 1; }
+// whether it does so in blocks where no window slides
+__host__ __device__ constexpr bool attn_rows_lone(int G, int s_max) {
+  return G <= 2 && s_max > 1 && s_max < 16 / G;
 }
 
 // token metadata shared by the attention and merge kernels
@@ -223,21 +232,13 @@ __global__ __launch_bounds__(256) void k_attn_prep(PrepArgs a) {
 
 // ---------------------------------------------------------------------------
 // flash attention: one wave per (token, kv head, split); G query heads share
-// the kv head (G <= 16).
+// the kv head (G <= 16).  wsh: the wave's LDS for 16 x G weights [p][head].
 // ---------------------------------------------------------------------------
 template <int HD, int G>
-__global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
+__device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int kvh, int s,
+                                                float* wsh) {
   constexpr int C = HD / 64;  // 64-byte K chunks per row = V bytes per lane
-  const int wave = threadIdx.x >> 6, lane = lane_id();
-  __shared__ __attribute__((aligned(16))) float s_w[4][16 * G];  // per wave: weights [p][head]
-  float* wsh = s_w[wave];
-  const int per_tok = a.num_kv * a.s_max;
-  const int item = blockIdx.x * 4 + wave;
-  if (item >= a.T * per_tok) return;
-  // later buffer rows first: in a prefill chunk they have the longest KV
-  // ranges, so the long waves start early and the short ones fill the tail
-  const int tok = a.T - 1 - item / per_tok, rem = item % per_tok;
-  const int kvh = rem / a.s_max, s = rem % a.s_max;
+  const int lane = lane_id();
   const TokRange tr = token_range(a, tok);
   const int S = num_splits(tr.L, a.s_max);
   if (s >= S) return;
@@ -296,11 +297,13 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
   float m[4], l[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) { m[i] = -1e30f; l[i] = 0.0f; }
-  float acc[G][C];
+  // acc[h / 4][c][h % 4]: head h, column lane * C + c
+  constexpr int HB = (G + 3) / 4;
+  v4f acc[HB][C];
 #pragma unroll
-  for (int h = 0; h < G; ++h)
+  for (int b = 0; b < HB; ++b)
 #pragma unroll
-    for (int c = 0; c < C; ++c) acc[h][c] = 0.0f;
+    for (int c = 0; c < C; ++c) acc[b][c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
   const int8_t* kbase = a.k_cache + (int64_t)kvh * HD;
   const int8_t* vbase = a.v_cache + (int64_t)kvh * HD + lane * C;
@@ -312,55 +315,67 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
   };
   // One tile's operands: lane (p + 16 g) holds K row p's bytes [c*64 + g*16,
   // +16) for every chunk c, its ks and vs; every lane holds its C bytes of
-  // each V row.  Idle positions repeat the tile's first row.
-  struct Tile {
-    v4i kb[C];
-    uint32_t vraw[16][(C + 3) / 4];
-    float ks, vs;
-  };
-  auto load_tile = [&](Tile& t, int p0, int slots, int sb) {
-    const int tl = end - p0 < 16 ? end - p0 : 16;
-    const int off = p0 - sb;
+  // each V row.  Idle positions repeat the tile's first row.  Up to two heads,
+  // each register is requested again, for the next tile, as soon as this tile
+  // has used it (AHEAD): a wave waits for memory once, not once per tile.  With
+  // more heads the registers this takes cost more than the wait (16 sequences
+  // of 4096 positions, head 512: the block 91 -> 111 us).
+  constexpr bool AHEAD = G <= 2;
+  v4i kb[C];
+  uint32_t vraw[16][(C + 3) / 4];
+  float ks, vs;
+  auto load_k = [&](int slots, int off, int tl) {
     const int my = __shfl(slots, off + (p16 < tl ? p16 : 0), kWave);
     const int8_t* krow = kbase + (int64_t)my * kvs + grp * 16;
 #pragma unroll
-    for (int c = 0; c < C; ++c) t.kb[c] = ld16(krow + c * 64);
-    t.ks = a.k_scale[(int64_t)my * a.num_kv + kvh];
-    t.vs = a.v_scale[(int64_t)my * a.num_kv + kvh];
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-      {
-        const int sp = __builtin_amdgcn_readlane(slots, off + (p < tl ? p : 0));
-        const int8_t* vr = vbase + (int64_t)sp * kvs;
-        if constexpr (C >= 8) {
-          const uint2 w = *reinterpret_cast<const uint2*>(vr);
-          t.vraw[p][0] = w.x; t.vraw[p][1] = w.y;
-        } else if constexpr (C == 4) {
-          t.vraw[p][0] = *reinterpret_cast<const uint32_t*>(vr);
-        } else if constexpr (C == 2) {
-          t.vraw[p][0] = *reinterpret_cast<const uint16_t*>(vr);
-        } else {
-          t.vraw[p][0] = (uint8_t)*vr;
-        }
-      }
+    for (int c = 0; c < C; ++c) kb[c] = ld16(krow + c * 64);
+    ks = a.k_scale[(int64_t)my * a.num_kv + kvh];
+    vs = a.v_scale[(int64_t)my * a.num_kv + kvh];
+  };
+  auto load_v = [&](int p, int slots, int off, int tl) {
+    const int sp = __builtin_amdgcn_readlane(slots, off + (p < tl ? p : 0));
+    const int8_t* vr = vbase + (int64_t)sp * kvs;
+    if constexpr (C >= 8) {
+      const uint2 w = *reinterpret_cast<const uint2*>(vr);
+      vraw[p][0] = w.x; vraw[p][1] = w.y;
+    } else if constexpr (C == 4) {
+      vraw[p][0] = *reinterpret_cast<const uint32_t*>(vr);
+    } else if constexpr (C == 2) {
+      vraw[p][0] = *reinterpret_cast<const uint16_t*>(vr);
+    } else {
+      vraw[p][0] = (uint8_t)*vr;
     }
   };
 
-  // (loading the next tile before this tile's arithmetic measured no faster:
-  // the kernel is bound by VALU issue once several waves share a SIMD)
-  Tile cur;
-  int sb = start, slots = 0;
-  if (start < end) slots = slot_batch(sb);
+  int off = 0, slots = 0, slots_n = 0;  // the next tile: its batch, and the batch after
+  if (start < end) {
+    slots = slot_batch(start);
+    slots_n = slot_batch(start + 64);
+    if constexpr (AHEAD) {
+      load_k(slots, 0, end - start);
+#pragma unroll
+      for (int p = 0; p < 16; ++p) load_v(p, slots, 0, end - start);
+    }
+  }
   for (int p0 = start; p0 < end; p0 += 16) {
     const int tl = end - p0 < 16 ? end - p0 : 16;
-    if (p0 - sb >= 64) {
-      sb = p0;
-      slots = slot_batch(sb);
+    const int tl_n = end - p0 - 16;  // of the next tile; <= 0: there is none
+    if constexpr (!AHEAD) {
+      load_k(slots, off, tl);
+#pragma unroll
+      for (int p = 0; p < 16; ++p) load_v(p, slots, off, tl);
     }
-    load_tile(cur, p0, slots, sb);
+    off += 16;
+    if (off == 64) {
+      off = 0;
+      slots = slots_n;
+      slots_n = slot_batch(p0 + 80);
+    }
     v4i d = zero4;
 #pragma unroll
-    for (int c = 0; c < C; ++c) d = mfma16x16x64(qa[c], cur.kb[c], d);
+    for (int c = 0; c < C; ++c) d = mfma16x16x64(qa[c], kb[c], d);
+    const float ks_t = ks, vs_t = vs;
+    if (AHEAD && tl_n > 0) load_k(slots, off, tl_n);
     const int dv[4] = {d.x, d.y, d.z, d.w};
     // per head of this lane's group (heads 4 g + i, only i < G exist)
     constexpr int NI = G < 4 ? G : 4;
@@ -369,56 +384,64 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
     for (int i = 0; i < NI; ++i) {
       float sco = -1e30f;
       if (4 * grp + i < G && p16 < tl)
-        sco = (((float)(dv[i] + qsum128[i]) - qb[i]) * fq[i]) * cur.ks * inv127sq;
+        sco = (((float)(dv[i] + qsum128[i]) - qb[i]) * fq[i]) * ks_t * inv127sq;
       const float tmax = group_max(sco, 16);
       const float m_new = tmax > m[i] ? tmax : m[i];
       corr[i] = fast_exp_softmax_biased(max87(m[i] - m_new));
       const float w = fast_exp_softmax_biased(max87(sco - m_new));
       l[i] = l[i] * corr[i] + tree16(w);
       m[i] = m_new;
-      sc[i] = p16 < tl ? w * cur.vs * inv127 : 0.0f;
+      sc[i] = p16 < tl ? w * vs_t * inv127 : 0.0f;
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
       const float ch = readlane_f(corr[h % 4], 16 * (h / 4));
 #pragma unroll
-      for (int c = 0; c < C; ++c) acc[h][c] = acc[h][c] * ch;
+      for (int c = 0; c < C; ++c) acc[h / 4][c][h % 4] = acc[h / 4][c][h % 4] * ch;
     }
     // positions past the tile's end carry weight 0: acc + v*0 leaves acc
     // unchanged bit for bit (acc is never -0: it starts at +0 and only an
     // exact -0 product added to -0 gives -0), so the loop needs no branch.
-    // The weights go through LDS as [p][head] and are read broadcast.
+    // The weights go through LDS, from G = 4 as [p][head % 4][head / 4]: lane
+    // L reads those of heads L % 4, + 4, ..., the MFMA's rows (a row of four
+    // fmaf in 2.3 cycles a lane against 2.6 to 4.2 for each v_fma); else as
+    // [p][head], read broadcast.
     if constexpr (G >= 4) {
 #pragma unroll
       for (int i = 0; i < NI; ++i)
-        if (4 * grp + i < G) wsh[p16 * G + 4 * grp + i] = sc[i];
+        if (4 * grp + i < G) wsh[p16 * G + i * HB + grp] = sc[i];
     } else {
 #pragma unroll
       for (int i = 0; i < NI; ++i)
         if (grp == 0) wsh[p16 * G + i] = sc[i];
     }
+    auto update = [&](auto reload) {
 #pragma unroll
-    for (int p = 0; p < 16; ++p) {
-      float vf[C];
+      for (int p = 0; p < 16; ++p) {
+        float vf[C];
 #pragma unroll
-      for (int c = 0; c < C; ++c)
-        vf[c] = (float)(int8_t)(cur.vraw[p][c / 4] >> (8 * (c % 4)));
-      float w[G];
-      if constexpr (G >= 4) {
+        for (int c = 0; c < C; ++c) vf[c] = (float)(int8_t)(vraw[p][c / 4] >> (8 * (c % 4)));
+        if constexpr (decltype(reload)::value) load_v(p, slots, off, tl_n);
+        if constexpr (G >= 4) {
+          float w[HB];
 #pragma unroll
-        for (int h4 = 0; h4 < G / 4; ++h4) {
-          const float4 w4 = *reinterpret_cast<const float4*>(&wsh[p * G + 4 * h4]);
-          w[4 * h4] = w4.x; w[4 * h4 + 1] = w4.y; w[4 * h4 + 2] = w4.z; w[4 * h4 + 3] = w4.w;
+          for (int b = 0; b < HB; ++b) w[b] = wsh[p * G + (lane & 3) * HB + b];
+#pragma unroll
+          for (int b = 0; b < HB; ++b)
+#pragma unroll
+            for (int c = 0; c < C; ++c) acc[b][c] = mfma4x64x1f(w[b], vf[c], acc[b][c]);
+        } else {
+#pragma unroll
+          for (int h = 0; h < G; ++h) {
+            const float w = wsh[p * G + h];
+#pragma unroll
+            for (int c = 0; c < C; ++c) acc[0][c][h] = fmaf(vf[c], w, acc[0][c][h]);
+          }
         }
-      } else {
-#pragma unroll
-        for (int h = 0; h < G; ++h) w[h] = wsh[p * G + h];
       }
-#pragma unroll
-      for (int h = 0; h < G; ++h)
-#pragma unroll
-        for (int c = 0; c < C; ++c) acc[h][c] = fmaf(vf[c], w[h], acc[h][c]);
-    }
+    };
+    if (AHEAD && tl_n > 0) update(std::true_type{});
+    else update(std::false_type{});
   }
 
   // finished here: a sliding token with one split (acc * (1/l)), and every
@@ -435,13 +458,15 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
       if (a.window > 0) {
         const float inv_l = lh > 0.0f ? 1.0f / lh : 0.0f;
 #pragma unroll
-        for (int c = 0; c < C; ++c) o[c] = lh > 0.0f ? f32_to_bf16(acc[h][c] * inv_l) : 0;
+        for (int c = 0; c < C; ++c)
+          o[c] = lh > 0.0f ? f32_to_bf16(acc[h / 4][c][h % 4] * inv_l) : 0;
       } else {
         const float cm = lh > 0.0f ? fast_exp_softmax_biased(0.0f) : 0.0f;
         const float gl = 0.0f + lh * cm;
         const float inv_l = gl > 0.0f ? 1.0f / gl : 0.0f;
 #pragma unroll
-        for (int c = 0; c < C; ++c) o[c] = gl > 0.0f ? f32_to_bf16((acc[h][c] * cm) * inv_l) : 0;
+        for (int c = 0; c < C; ++c)
+          o[c] = gl > 0.0f ? f32_to_bf16((acc[h / 4][c][h % 4] * cm) * inv_l) : 0;
       }
       uint16_t* dst = a.out + qrow * HD + lane * C;
 #pragma unroll
@@ -449,7 +474,7 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
     } else {
       float* pa = a.ws_acc + (qrow * a.s_max + s) * HD + lane * C;
 #pragma unroll
-      for (int c = 0; c < C; ++c) pa[c] = acc[h][c];
+      for (int c = 0; c < C; ++c) pa[c] = acc[h / 4][c][h % 4];
       if (lane == 0) {
         a.ws_ml[(qrow * a.s_max + s) * 2 + 0] = mh;
         a.ws_ml[(qrow * a.s_max + s) * 2 + 1] = lh;
@@ -458,265 +483,397 @@ __global__ __launch_bounds__(256) void k_flash_attn(AttnArgs a) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Single-split tokens (s_max == 1, prefill chunks): TPW = 16 / G query tokens
-// per wave share every K/V tile.  The wave takes the tokens tok0 + 16 k
-// (k < TPW) of one run: their ranges start at positions that are equal mod 16
-// (sliding: lo = pos - window + 1 once pos >= window - 1, else 0; full: 0),
-// so all their 16-position tiles sit on one grid and a tile of the grid is,
-// for each token, either one of its own tiles or outside its range.  Rows of
-// the MFMA are (token k, head h) = 16 rows; each row keeps its own m, l, acc
-// and runs the reference's tile recursion; the V conversion and the K/V loads
-// are shared by the 16 rows.  Tokens that do not share a grid (a group that
-// straddles pos = window - 1, or spans two runs) are processed one per pass.
-// Results are those of the one-split path: acc * (1/l) for sliding layers,
-// the one-split merge ((acc * c) * (1/(l * c)), c = fast_exp(0)) for full.
-// ---------------------------------------------------------------------------
 template <int HD, int G>
-__global__ __launch_bounds__(256) void k_flash_attn_mt(AttnArgs a) {
-  constexpr int C = HD / 64, TPW = 16 / G;
-  const int wave = threadIdx.x >> 6, lane = lane_id();
-  __shared__ __attribute__((aligned(16))) float s_w[4][16 * 16];  // per wave: weights [p][row]
-  const int nblk = (a.T + 16 * TPW - 1) / (16 * TPW);
+__global__ __launch_bounds__(256, 2) void k_flash_attn(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float s_w[4][16 * G];
+  const int wave = threadIdx.x >> 6;
+  const int per_tok = a.num_kv * a.s_max;
   const int item = blockIdx.x * 4 + wave;
-  if (item >= nblk * a.num_kv * 16) return;
-  // later token blocks first (the longest KV ranges of a prefill chunk)
-  const int cls = item % 16, kvh = (item / 16) % a.num_kv;
-  const int blk = nblk - 1 - item / (16 * a.num_kv);
-  const int tok0 = blk * 16 * TPW + cls;
-  const int64_t kvs = (int64_t)a.num_kv * HD;
+  if (item >= a.T * per_tok) return;
+  // later buffer rows first: in a prefill chunk they have the longest KV
+  // ranges, so the long waves start early and the short ones fill the tail
+  const int tok = a.T - 1 - item / per_tok, rem = item % per_tok;
+  flash_attn_wave<HD, G>(a, tok, rem / a.s_max, rem % a.s_max, s_w[wave]);
+}
+
+// ---------------------------------------------------------------------------
+// Row-group attention: one workgroup of four waves per (16 / G query tokens,
+// kv head, split).  The group's 16 (token, head) rows are the rows of every
+// MFMA, and each step of the workgroup takes four of the reference's
+// 16-position tiles.
+//   A  wave w scores tile w (int8 MFMA, K rows from memory), and its tile
+//      maxima go to LDS; after a barrier every row's running maximum, the
+//      tile's correction, weights and 16-lane weight sum follow, and go to LDS.
+//   B  after a second barrier every wave applies the four tiles, in order, to
+//      its quarter of the head's columns: acc *= corr, then acc += w * v by
+//      f32 MFMA, whose products are exactly the reference's fmaf chain over
+//      the positions (mfma16x16x4f).
+// Rows keep their own m, l and acc and the reference's tile recursion, which
+// needs tiles counted from the row's own first position: tokens of one run
+// whose ranges start equal mod 16 are one set, on one tile grid; the tiles of
+// a group's sets follow each other.  A row outside a tile has corr 1 and
+// weights 0, which leave its acc (never -0) bit for bit.
+// It is bound by instruction issue: the f32 MFMA runs on the vector ALU's own
+// multipliers (33 cycles for 1024 fmaf per SIMD, and none of another wave's
+// vector work beside it), so a step of head 256 costs 64 of them plus about
+// 400 vector instructions per wave.  The block of 2048 tokens from position 0
+// (sliding, head 256): 598 -> 412 us, attention alone 403 -> 222 us against a
+// wave per 8 tokens on v_fma; 700 + 411 tokens (full, head 512): 699 -> 396 us.
+template <int HD, int G>
+__global__ __launch_bounds__(256, HD >= 512 ? 2 : 3) void k_flash_attn_rows(AttnArgs a, int nblk) {
+  constexpr int C = HD / 64;    // 64-byte K chunks per row; column tiles per wave
+  constexpr int TPW = 16 / G;   // tokens per group
+  constexpr int NL = G >= 4 ? 1 : 4 / G;  // tokens among a lane's four rows
+  constexpr int NH = attn_rows_parts(G);  // workgroups per group
+  // a step's weights [position][row]; corrections, weight sums (row 4: a spare)
+  // and maxima [tile][row]
+  __shared__ __attribute__((aligned(16))) float s_w[64 * 16];
+  __shared__ __attribute__((aligned(16))) float s_corr[4][16], s_sum[5][16], s_tm[4][16];
+  __shared__ __attribute__((aligned(16))) float s_mn[4][16];  // per wave: its tile's new maxima
+  __shared__ __attribute__((aligned(16))) int8_t s_q[C][1024];  // the A operands, by lane
+  __shared__ __attribute__((aligned(16))) float s_qb[16], s_fq[16];  // per row
+  __shared__ __attribute__((aligned(16))) int s_qs[16];
+  __shared__ uint64_t s_row[4][64];  // per wave: the step's cache row offsets
+  __shared__ int s_set[TPW][4];      // sets: first position, end, page table offset, first tile
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
   const int p16 = lane & 15, grp = lane >> 4;
-
-  // per-token range (wave-uniform): run, [lo, hi) of positions
-  int run_k[TPW];
-  int lo_k[TPW], hi_k[TPW];  // positions fit in 32 bits
-  bool shared = true;
+  // kv head fastest (workgroups go round the XCDs, so an XCD's L2 sees few kv
+  // heads), then split, then the block's groups; later tokens first: in a
+  // prefill chunk they have the longest ranges, and the short ones fill the tail
+  int item = blockIdx.x;
+  const int kvh = item % a.num_kv;
+  item /= a.num_kv;
+  const int s = item % a.s_max;
+  item /= a.s_max;
+  // (the parts come last: where one alone has work, workgroups without any
+  // between it would leave some shader engines idle)
+  const int part = item / (nblk * 16);
+  item -= part * nblk * 16;
+  const int cls = item % 16, t0 = (nblk - 1 - item / 16) * 16 * TPW;
+  const int run0 = run_of(a.runs, a.num_runs, t0);
+  auto run_from = [&](int tok) {  // run_of(tok), tok >= t0
+    int r = run0;
+    while (r + 1 < a.num_runs && tok >= a.runs[r + 1].buf_start) ++r;
+    return r;
+  };
+  // groups take tokens 16 apart where some window of the block slides (equal
+  // starts mod 16), and neighbours where every range starts at position 0 (no
+  // tile of one is past the other)
+  int tok0 = t0 + cls * TPW, step = 1;
+  if (a.window > 0) {
+    bool slides = false;
 #pragma unroll
-  for (int k = 0; k < TPW; ++k) {
-    const int tok = tok0 + 16 * k;
-    run_k[k] = -1; lo_k[k] = 0; hi_k[k] = 0;
-    if (tok >= a.T) continue;
-    const TokRange tr = token_range(a, tok);
-    run_k[k] = run_of(a.runs, a.num_runs, tok);
-    lo_k[k] = (int)tr.lo;
-    hi_k[k] = (int)tr.lo + tr.L;
-    if (run_k[k] != run_k[0] || ((lo_k[k] - lo_k[0]) & 15) != 0) shared = false;
+    for (int q = 0; q < 16 * TPW; q += kWave) {
+      const int tok = t0 + q + lane;
+      if (q + lane < 16 * TPW && tok < a.T) {
+        const KvRun run = a.runs[run_from(tok)];
+        slides |= run.base_pos + (tok - run.buf_start) >= a.window;
+      }
+    }
+    if (__ballot(slides)) { tok0 = t0 + cls; step = 16; }
+  }
+  if constexpr (NH > 1) {
+    // Where nothing slides, two neighbours' splits start together only if
+    // ceil(L / S) is the same for both: with fewer splits than tokens a group
+    // would be several small sets, and a wave per token is faster (200 tokens
+    // from position 0, two splits: the block 83 against 74 us)
+    if (step == 1 && attn_rows_lone(G, a.s_max)) {
+      const int tok = tok0 + 4 * part + wave;
+      if (tok < a.T) flash_attn_wave<HD, G>(a, tok, kvh, s, s_w + wave * 16 * G);
+      return;
+    }
+    if (part > 0) return;
+  }
+  if (tok0 >= a.T) return;
+  const int64_t kvs = (int64_t)a.num_kv * HD;
+
+  // token lane % TPW of the group: its positions [t_beg, t_end) of this split,
+  // its number of splits (0: no token), its set
+  int t_beg = 0, t_end = 0, t_S, t_set = -1, nsets = 0, tiles = 0;
+  {
+    const int tok = tok0 + step * (lane % TPW);
+    const int r = run_from(tok);
+    const KvRun run = a.runs[r];
+    const int pos = run.base_pos + (tok - run.buf_start);
+    const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
+    const int L = pos + 1 - lo;  // <= 0: no positions
+    t_S = num_splits(L, a.s_max);
+    const int per = (L + t_S - 1) / t_S;
+    if (tok < a.T && s < t_S && s * per < L) {
+      t_beg = lo + s * per;
+      t_end = lo + (s * per + per < L ? s * per + per : L);
+    }
+    if (tok >= a.T) t_S = 0;
+    if (!__ballot(s < t_S)) return;  // no token has this split
+    unsigned todo = (unsigned)__ballot(lane < TPW && t_end > t_beg);
+    for (; todo; ++nsets) {  // uniform; every wave makes the same table
+      const int f = __ffs((int)todo) - 1;
+      const bool in = ((todo >> (lane % TPW)) & 1u) && r == __builtin_amdgcn_readlane(r, f) &&
+                      ((t_beg - __builtin_amdgcn_readlane(t_beg, f)) & 15) == 0;
+      if (in) t_set = nsets;
+      todo &= ~(unsigned)__ballot(lane < TPW && in);
+      int pbeg = in ? t_beg : 0x7FFFFFFF, pend = in ? t_end : 0;
+#pragma unroll
+      for (int o = 1; o < TPW; o <<= 1) {
+        pbeg = min(pbeg, __shfl_xor(pbeg, o, kWave));
+        pend = max(pend, __shfl_xor(pend, o, kWave));
+      }
+      if (lane == 0) {
+        s_set[nsets][0] = pbeg;
+        s_set[nsets][1] = pend;
+        s_set[nsets][2] = __builtin_amdgcn_readlane(run.rows_off, f);
+        s_set[nsets][3] = tiles;
+      }
+      tiles += (__builtin_amdgcn_readfirstlane(pend) - __builtin_amdgcn_readfirstlane(pbeg) + 15) >> 4;
+    }
   }
 
-  // A operand: row r = k * G + h (token k, head h); lane (r + 16 g) holds
-  // row r's bytes [c*64 + g*16, +16)
+  // A operand: row r = k * G + h (token k, head h); lane (r + 16 g) holds row
+  // r's bytes [c*64 + g*16, +16).  Scores: lane (p + 16 g), value i <-> row
+  // 4 g + i, position p.
   const v4i zero4 = {0, 0, 0, 0};
-  v4i qa[C];
   {
-    const int r = lane & 15, k = r / G, h = r % G;
-    const int tok = tok0 + 16 * k;
-    const int8_t* qrow = a.q_i8 + ((int64_t)(tok < a.T ? tok : 0) * a.num_q + kvh * G + h) * HD +
-                         grp * 16;
-#pragma unroll
-    for (int c = 0; c < C; ++c) qa[c] = tok < a.T ? ld16(qrow + c * 64) : zero4;
-  }
-  // score layout: lane (p + 16 g), value i <-> row 4 g + i
-  float qb[4], fq[4];
-  int qsum128[4];
-  {
+    const int tok = min(tok0 + step * (p16 / G), a.T - 1);  // (rows without a token: never used)
+    const int64_t qrow = (int64_t)tok * a.num_q + kvh * G + p16 % G;
     int part = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const int w4[4] = {qa[c].x, qa[c].y, qa[c].z, qa[c].w};
+      const v4i q = ld16(a.q_i8 + qrow * HD + c * 64 + grp * 16);
+      const int w4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        part += (int)(int8_t)w4[q] + (int)(int8_t)(w4[q] >> 8) + (int)(int8_t)(w4[q] >> 16) +
-                (w4[q] >> 24);
+      for (int j = 0; j < 4; ++j)
+        part += (int)(int8_t)w4[j] + (int)(int8_t)(w4[j] >> 8) + (int)(int8_t)(w4[j] >> 16) +
+                (w4[j] >> 24);
+      if (c % 4 == wave) *reinterpret_cast<v4i*>(&s_q[c][lane * 16]) = q;
     }
     part += __shfl_xor(part, 16, kWave);
     part += __shfl_xor(part, 32, kWave);  // lane r (and r + 16 g): sum of row r's codes
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 4 * grp + i, k = r / G, h = r % G, tok = tok0 + 16 * k;
-      qsum128[i] = 128 * __shfl(part, r, kWave);
-      qb[i] = 0.0f; fq[i] = 0.0f;
-      if (tok < a.T) {
-        qb[i] = a.qi_bias[(int64_t)tok * a.num_q + kvh * G + h];
-        fq[i] = a.f_q[(int64_t)tok * a.num_q + kvh * G + h];
-      }
+    if (wave == 0 && lane < 16) {
+      s_qs[lane] = 128 * part;  // the u8-shifted dot of the reference is dot + 128 * sum(q)
+      s_qb[lane] = a.qi_bias[qrow];
+      s_fq[lane] = a.f_q[qrow];
     }
   }
+  lds_barrier();
+
+  // positions of this lane's rows 4 grp + i, and of row p16, and their sets
+  int lo[NL], hi[NL], rs[NL];
+#pragma unroll
+  for (int t = 0; t < NL; ++t) {
+    const int k = 4 * grp / G + t;
+    lo[t] = __shfl(t_beg, k, kWave);
+    hi[t] = __shfl(t_end, k, kWave);
+    rs[t] = __shfl(t_set, k, kWave);
+  }
+  const int lo_r = __shfl(t_beg, p16 / G, kWave), hi_r = __shfl(t_end, p16 / G, kWave);
+  const int rs_r = __shfl(t_set, p16 / G, kWave);
 
   const float inv127 = 1.0f / 127.0f;
   const float inv127sq = inv127 * inv127;
-  float m[4], l[4];
-  float acc[16][C];
+  float m = -1e30f, l = 0.0f;  // row p16's running maximum and sum
+  v4f acc[C];                  // columns (wave * 16 + p16) * C + ct, rows 4 grp + i
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { m[i] = -1e30f; l[i] = 0.0f; }
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-#pragma unroll
-    for (int c = 0; c < C; ++c) acc[r][c] = 0.0f;
-  const int8_t* kbase = a.k_cache + (int64_t)kvh * HD;
-  const int8_t* vbase = a.v_cache + (int64_t)kvh * HD + lane * C;
+  for (int c = 0; c < C; ++c) acc[c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  const int8_t* kbase = a.k_cache + (int64_t)kvh * HD + grp * 16;
+  const int8_t* vbase = a.v_cache + (int64_t)kvh * HD + (wave * 16 + p16) * C;
 
-  // one pass over all tokens (shared grid) or one pass per token
-  const int npass = shared ? 1 : TPW;
-  for (int pass = 0; pass < npass; ++pass) {
-    // active tokens of this pass and the position range they cover
-    unsigned amask = 0;
-    int pbeg = 0, pend = 0;
-    int run = -1;
+  // Tile n0 + grp of the list: its set (-1 past the last tile), its first
+  // position and the slot of its position p16 (those past the set's end, or
+  // the list's, repeat a position: their weights are 0).
+  int n_set = 0, n_pos = 0, slot = 0;
+  auto next_tiles = [&](int n0) {
+    const int n = min(n0 + grp, tiles - 1);
+    int c = n_set < 0 ? nsets - 1 : n_set;
+    while (c + 1 < nsets && n >= s_set[c + 1][3]) ++c;
+    const int beg = s_set[c][0] + 16 * (n - s_set[c][3]);
+    const int p = min(beg + p16, s_set[c][1] - 1);
+    slot = (int)paged_slot(a.base_rows + s_set[c][2], a.page_shift, a.row_mask, a.page_mask, p);
+    n_set = n0 + grp < tiles ? c : -1;
+    n_pos = beg;
+  };
+  v4i kb[C];
+  float ks, vs;
+  auto load_k = [&]() {  // K rows of tile `wave`; all rows' byte offsets through LDS
+    // (a wave's own LDS accesses are in order: no barrier)
+    s_row[wave][lane] = (uint64_t)(uint32_t)slot * (uint32_t)kvs;
+    const int64_t my = __shfl(slot, 16 * wave + p16, kWave);
+    const int8_t* kr = kbase + s_row[wave][16 * wave + p16];
 #pragma unroll
-    for (int k = 0; k < TPW; ++k) {
-      const bool on = run_k[k] >= 0 && (shared || k == pass) && hi_k[k] > lo_k[k];
-      if (!on) continue;
-      if (amask == 0) { pbeg = lo_k[k]; pend = hi_k[k]; run = run_k[k]; }
-      pbeg = lo_k[k] < pbeg ? lo_k[k] : pbeg;
-      pend = hi_k[k] > pend ? hi_k[k] : pend;
-      amask |= 1u << k;
+    for (int c = 0; c < C; ++c) kb[c] = ld16(kr + c * 64);
+    ks = a.k_scale[my * a.num_kv + kvh];
+    vs = a.v_scale[my * a.num_kv + kvh];
+  };
+  if (tiles > 0) {
+    next_tiles(0);
+    load_k();
+  }
+  for (int n0 = 0; n0 < tiles; n0 += 4) {
+    const int set = n_set, pos = n_pos;  // of tile n0 + grp
+    // this step's V: lane (j + 16 k) holds C bytes of position 4 u + k
+    uint32_t vraw[16][(C + 3) / 4];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int8_t* vr = vbase + s_row[wave][4 * u + grp];
+      if constexpr (C == 8) {
+        const uint2 w = *reinterpret_cast<const uint2*>(vr);
+        vraw[u][0] = w.x; vraw[u][1] = w.y;
+      } else if constexpr (C == 4) {
+        vraw[u][0] = *reinterpret_cast<const uint32_t*>(vr);
+      } else if constexpr (C == 2) {
+        vraw[u][0] = *reinterpret_cast<const uint16_t*>(vr);
+      } else {
+        vraw[u][0] = (uint8_t)*vr;
+      }
     }
-    if (amask == 0) continue;
-    const int32_t* rows = a.base_rows + a.runs[run].rows_off;
-    for (int P = pbeg; P < pend; P += 16) {
-      // rows taking part in this tile, and their tile lengths
-      unsigned rmask = 0;
-      int tl_k[TPW];
+    next_tiles(n0 + 4);
+    // ---- A: scores of tile `wave` -------------------------------------------
+    const int w_set = __builtin_amdgcn_readlane(set, 16 * wave);
+    const int w_pos = __builtin_amdgcn_readlane(pos, 16 * wave);
+    v4i d = zero4;
 #pragma unroll
-      for (int k = 0; k < TPW; ++k) {
-        tl_k[k] = 0;
-        if (!((amask >> k) & 1u) || P < lo_k[k] || P >= hi_k[k]) continue;
-        tl_k[k] = hi_k[k] - P < 16 ? hi_k[k] - P : 16;
-        rmask |= ((1u << G) - 1u) << (k * G);
+    for (int c = 0; c < C; ++c)
+      d = mfma16x16x64(*reinterpret_cast<const v4i*>(&s_q[c][lane * 16]), kb[c], d);
+    const v4i qs4 = *reinterpret_cast<const v4i*>(&s_qs[4 * grp]);
+    const v4f qb4 = *reinterpret_cast<const v4f*>(&s_qb[4 * grp]);
+    const v4f fq4 = *reinterpret_cast<const v4f*>(&s_fq[4 * grp]);
+    float sco[4], tm[4];
+    bool on[4], ok[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = NL == 1 ? 0 : i / (4 / NL);
+      const bool in = rs[t] == w_set && w_pos >= lo[t];
+      on[i] = in && w_pos < hi[t];
+      ok[i] = in && w_pos + p16 < hi[t];
+      sco[i] = (((float)(d[i] + qs4[i]) - qb4[i]) * fq4[i]) * ks * inv127sq;
+      sco[i] = ok[i] ? sco[i] : -1e30f;
+      tm[i] = sco[i];
+    }
+    row_max16_x4(tm);
+    const float vs_t = vs;
+    *reinterpret_cast<float4*>(&s_tm[wave][4 * grp]) = float4{tm[0], tm[1], tm[2], tm[3]};
+    lds_barrier();
+    // row p16, tile grp: the running maximum before and after the tile, and
+    // the correction (every wave the same; 1 where the row is outside the tile)
+    {
+      const float x0 = s_tm[0][p16], x1 = s_tm[1][p16], x2 = s_tm[2][p16], x3 = s_tm[3][p16];
+      const float a0 = max_num(m, x0), a1 = max_num(a0, x1), a2 = max_num(a1, x2);
+      const float a3 = max_num(a2, x3);
+      const float before = grp < 2 ? (grp == 0 ? m : a0) : (grp == 2 ? a1 : a2);
+      const float after = grp < 2 ? (grp == 0 ? a0 : a1) : (grp == 2 ? a2 : a3);
+      const float cr = fast_exp_softmax_le0(max_num(before - after, -87.0f));
+      s_corr[grp][p16] = rs_r == set && pos >= lo_r && pos < hi_r ? cr : 1.0f;
+      if (grp == wave) s_mn[wave][p16] = after;
+      m = a3;
+    }
+    const v4f mn = *reinterpret_cast<const v4f*>(&s_mn[wave][4 * grp]);
+    float wt[4], sum[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float w = fast_exp_softmax_le0(max_num(sco[i] - mn[i], -87.0f));
+      const float t = row_tree16(w);  // in lane 0 of the row
+      sum[i] = on[i] ? t : 0.0f;
+      wt[i] = ok[i] ? w * vs_t * inv127 : 0.0f;
+    }
+    *reinterpret_cast<float4*>(&s_w[(16 * wave + p16) * 16 + 4 * grp]) =
+        float4{wt[0], wt[1], wt[2], wt[3]};
+    // (lanes without a sum write to the spare row: no branch)
+    *reinterpret_cast<float4*>(&s_sum[p16 == 0 ? wave : 4][4 * grp]) =
+        float4{sum[0], sum[1], sum[2], sum[3]};
+    load_k();
+    lds_barrier();
+    // ---- B: the tiles' updates of this wave's columns -----------------------
+    auto update = [&](int t) {
+      const v4f cv = *reinterpret_cast<const v4f*>(&s_corr[t][4 * grp]);
+      l = l * s_corr[t][p16] + s_sum[t][p16];
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[c][i] = acc[c][i] * cv[i];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int u = 4 * t + q;
+        const float w = s_w[(4 * u + grp) * 16 + p16];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          acc[c] = mfma16x16x4f(w, (float)(int8_t)(vraw[u][c / 4] >> (8 * (c % 4))), acc[c]);
       }
-      const int tlen = pend - P < 16 ? pend - P : 16;
-      const int pp = p16 < tlen ? p16 : 0;
-      const int slot = (int)paged_slot(rows, a.page_shift, a.row_mask, a.page_mask, P + pp);
-      v4i kb[C];
-      const int8_t* krow = kbase + (int64_t)slot * kvs + grp * 16;
+    };
+    if (n0 + 4 <= tiles) {
 #pragma unroll
-      for (int c = 0; c < C; ++c) kb[c] = ld16(krow + c * 64);
-      const float ks = a.k_scale[(int64_t)slot * a.num_kv + kvh];
-      const float vs = a.v_scale[(int64_t)slot * a.num_kv + kvh];
-      uint32_t vraw[16][(C + 3) / 4];
-#pragma unroll
-      for (int p = 0; p < 16; ++p) {
-        const int sp = __builtin_amdgcn_readlane(slot, p < tlen ? p : 0);
-        const int8_t* vr = vbase + (int64_t)sp * kvs;
-        if constexpr (C >= 8) {
-          const uint2 w = *reinterpret_cast<const uint2*>(vr);
-          vraw[p][0] = w.x; vraw[p][1] = w.y;
-        } else if constexpr (C == 4) {
-          vraw[p][0] = *reinterpret_cast<const uint32_t*>(vr);
-        } else if constexpr (C == 2) {
-          vraw[p][0] = *reinterpret_cast<const uint16_t*>(vr);
-        } else {
-          vraw[p][0] = (uint8_t)*vr;
-        }
-      }
-      v4i d = zero4;
-#pragma unroll
-      for (int c = 0; c < C; ++c) d = mfma16x16x64(qa[c], kb[c], d);
-      const int dv[4] = {d.x, d.y, d.z, d.w};
-      float sc[4], corr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * grp + i;
-        const bool on = (rmask >> r) & 1u;
-        // this row's tile length (lane-varying through the token index)
-        int tl = 0;
-#pragma unroll
-        for (int k = 0; k < TPW; ++k) tl = r / G == k ? tl_k[k] : tl;
-        float sco = -1e30f;
-        if (on && p16 < tl)
-          sco = (((float)(dv[i] + qsum128[i]) - qb[i]) * fq[i]) * ks * inv127sq;
-        const float tmax = group_max(sco, 16);
-        const float m_new = tmax > m[i] ? tmax : m[i];
-        const float cr = fast_exp_softmax_biased(max87(m[i] - m_new));
-        const float w = fast_exp_softmax_biased(max87(sco - m_new));
-        const float wsum = tree16(w);
-        corr[i] = on ? cr : 1.0f;
-        if (on) {
-          l[i] = l[i] * cr + wsum;
-          m[i] = m_new;
-        }
-        sc[i] = on && p16 < tl ? w * vs * inv127 : 0.0f;
-      }
-      // every row takes part in the update: a row outside this tile has
-      // corr 1 and weights 0, which leave its acc bit for bit (acc * 1 = acc,
-      // acc + v*0 = acc since acc is never -0), so the loops need no branches.
-      // The weights go through LDS as [p][row]; every lane reads them
-      // broadcast, four rows per read.
-      float* wsh = s_w[wave];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) wsh[p16 * 16 + 4 * grp + i] = sc[i];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float ch = readlane_f(corr[r % 4], 16 * (r / 4));
-#pragma unroll
-        for (int c = 0; c < C; ++c) acc[r][c] = acc[r][c] * ch;
-      }
-#pragma unroll
-      for (int p = 0; p < 16; ++p) {
-        float vf[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) vf[c] = (float)(int8_t)(vraw[p][c / 4] >> (8 * (c % 4)));
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const float4 w4 = *reinterpret_cast<const float4*>(&wsh[p * 16 + 4 * r4]);
-          const float wr[4] = {w4.x, w4.y, w4.z, w4.w};
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-              acc[4 * r4 + q][c] = fmaf(vf[c], wr[q], acc[4 * r4 + q][c]);
-        }
-      }
+      for (int t = 0; t < 4; ++t) update(t);
+    } else {  // a short last step
+      update(0);
+      if (n0 + 1 < tiles) update(1);
+      if (n0 + 2 < tiles) update(2);
     }
   }
 
-  // finalize every row of a real token
+  // finished here: a sliding token with one split (acc * (1/l)), and every
+  // token when the plan has one split (full layers: the merge of one split,
+  // (acc * c) * (1/(l * c)) with c = fast_exp(0)); other splits are partials
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int k = r / G, h = r % G, tok = tok0 + 16 * k;
-    if (tok >= a.T) continue;
-    const float lr = readlane_f(l[r % 4], 16 * (r / 4));
-    uint16_t o[C];
-    if (a.window > 0) {  // sliding prefill: acc * (1/l), or zeros
-      const float inv_l = lr > 0.0f ? 1.0f / lr : 0.0f;
-#pragma unroll
-      for (int c = 0; c < C; ++c) o[c] = lr > 0.0f ? f32_to_bf16(acc[r][c] * inv_l) : 0;
-    } else {             // the merge of one split
-      const float cm = lr > 0.0f ? fast_exp_softmax_biased(0.0f) : 0.0f;
-      const float gl = 0.0f + lr * cm;
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * grp + i, k = r / G, tok = tok0 + step * k;
+    const float lr = __shfl(l, r, kWave), mr = __shfl(m, r, kWave);
+    const int S = __shfl(t_S, k, kWave);
+    if (s >= S) continue;  // no such token, or no such split of it
+    const int64_t qrow = (int64_t)tok * a.num_q + kvh * G + r % G;
+    const int col = (wave * 16 + p16) * C;
+    if (S == 1 && (a.window > 0 || a.s_max == 1)) {
+      const float cm = a.window > 0 ? 1.0f : lr > 0.0f ? fast_exp_softmax_biased(0.0f) : 0.0f;
+      const float gl = a.window > 0 ? lr : 0.0f + lr * cm;
       const float inv_l = gl > 0.0f ? 1.0f / gl : 0.0f;
+      uint16_t* dst = a.out + qrow * HD + col;
 #pragma unroll
-      for (int c = 0; c < C; ++c) o[c] = gl > 0.0f ? f32_to_bf16((acc[r][c] * cm) * inv_l) : 0;
+      for (int c = 0; c < C; ++c) dst[c] = gl > 0.0f ? f32_to_bf16((acc[c][i] * cm) * inv_l) : 0;
+    } else {
+      float* pa = a.ws_acc + (qrow * a.s_max + s) * HD + col;
+#pragma unroll
+      for (int c = 0; c < C; ++c) pa[c] = acc[c][i];
+      if (wave == 0 && p16 == 0) {
+        a.ws_ml[(qrow * a.s_max + s) * 2 + 0] = mr;
+        a.ws_ml[(qrow * a.s_max + s) * 2 + 1] = lr;
+      }
     }
-    uint16_t* dst = a.out + ((int64_t)tok * a.num_q + kvh * G + h) * HD + lane * C;
-#pragma unroll
-    for (int c = 0; c < C; ++c) dst[c] = o[c];
   }
 }
 
 // ---------------------------------------------------------------------------
-// merge of the split partials: one wave per (token, query head)
+// merge of the split partials: one wave per (token, query head, 64 * CL
+// columns), CL columns per lane.  It is latency: a wave's rows (NB splits) are
+// all requested before the corrections are computed from the (m, l), and the
+// chain over the splits in order then runs from registers.
 // ---------------------------------------------------------------------------
-template <int HD>
+template <int HD, int NB, int CL>
 __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
-  // one wave per (token, query head, 128-column slice); lane owns CL columns
-  constexpr int CW = HD < 128 ? HD : 128, CL = CW / 64, NW = HD / CW;
+  constexpr int NW = HD / (64 * CL);
   const int wave = threadIdx.x >> 6, lane = lane_id();
   const int witem = blockIdx.x * 4 + wave;
   if (witem >= a.T * a.num_q * NW) return;
-  const int item = witem / NW, col0 = (witem % NW) * CW + lane * CL;
+  const int item = witem / NW, col = ((witem % NW) * 64 + lane) * CL;
   const int tok = item / a.num_q;
   const TokRange tr = token_range(a, tok);
   const int S = num_splits(tr.L, a.s_max);
   if (a.window > 0 && S == 1) return;  // finalized by the attention wave
   const int64_t base = (int64_t)item * a.s_max;
   const float* ml = a.ws_ml + base * 2;
+  const float* src = a.ws_acc + base * HD + col;
+  float rows[NB][CL];
+  auto load_rows = [&](int s0) {  // splits past S repeat the last (never used)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int j = 0; j < CL; ++j) rows[b][j] = src[(int64_t)min(s0 + b, S - 1) * HD + j];
+  };
   float gm = -1e30f;
   for (int s0 = 0; s0 < S; s0 += kWave) {
     const float v = s0 + lane < S ? ml[(s0 + lane) * 2] : -1e30f;
     gm = fmaxf(gm, wave_max(v));
   }
+  load_rows(0);
   float gl = 0.0f, out[CL];
+#pragma unroll
+  for (int j = 0; j < CL; ++j) out[j] = 0.0f;
   bool first = true;
   for (int s0 = 0; s0 < S; s0 += kWave) {
     // the corrections of 64 splits, lane-parallel; masked by l > 0
@@ -730,120 +887,26 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       if (s0 + 16 * q < S) gl = gl + readlane_f(bsum, 16 * q);
-    // acc: splits in order, 8 rows in flight
-    const int n = S - s0 < kWave ? S - s0 : kWave;
-    const float* src0 = a.ws_acc + (base + s0) * HD + col0;
-    for (int b0 = 0; b0 < n; b0 += 8) {
-      float rows[8][CL];
+    // acc: splits in order; those with a correction of 0 are left out, and the
+    // first of the others is multiplied
+    const unsigned long long live = __ballot(c > 0.0f);
 #pragma unroll
-      for (int b = 0; b < 8; ++b)
-        if (b0 + b < n) {
+    for (int h = 0; h < kWave; h += NB) {
+      if (s0 + h >= S) break;
+      if (s0 + h > 0) load_rows(s0 + h);
 #pragma unroll
-          for (int cc = 0; cc < CL; ++cc) rows[b][cc] = src0[(int64_t)(b0 + b) * HD + cc];
-        }
+      for (int b = 0; b < NB; ++b) {
+        if (!((live >> (h + b)) & 1ull)) continue;  // uniform
+        const float cb = readlane_f(c, h + b);
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        if (b0 + b >= n) break;
-        const float cb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), b0 + b));
-        if (cb <= 0.0f) continue;
-#pragma unroll
-        for (int cc = 0; cc < CL; ++cc)
-          out[cc] = first ? rows[b][cc] * cb : fmaf(rows[b][cc], cb, out[cc]);
+        for (int j = 0; j < CL; ++j) out[j] = first ? rows[b][j] * cb : fmaf(rows[b][j], cb, out[j]);
         first = false;
       }
     }
   }
-  uint16_t* dst = a.out + (int64_t)item * HD + col0;
-  if (!(gl > 0.0f)) {
-#pragma unroll
-    for (int cc = 0; cc < CL; ++cc) dst[cc] = 0;
-    return;
-  }
-  const float inv_l = 1.0f / gl;
-#pragma unroll
-  for (int cc = 0; cc < CL; ++cc) dst[cc] = f32_to_bf16(out[cc] * inv_l);
-}
-
-// Merge for many splits: one workgroup per (token, query head, 64-column
-// slice).  The four waves stage up to 240 splits (their (m, l) and the slice
-// of their acc rows) in LDS with all loads in flight at once; wave 0 then runs
-// the ordered chain from LDS, eight rows per batch.
-constexpr int kMergeStage = 240;  // 240 x 66 floats: under 64 KiB of LDS
-
-template <int HD>
-__global__ __launch_bounds__(256) void k_attn_merge_lds(AttnArgs a) {
-  constexpr int NW = HD / 64;
-  extern __shared__ float stage[];  // [n][64] acc slice, then [n] m, [n] l
-  const int wave = threadIdx.x >> 6, lane = lane_id();
-  const int item = blockIdx.x / NW, col = (blockIdx.x % NW) * 64 + lane;
-  const int tok = item / a.num_q;
-  const TokRange tr = token_range(a, tok);
-  const int S = num_splits(tr.L, a.s_max);
-  if (a.window > 0 && S == 1) return;  // finalized by the attention wave
-  const int64_t base = (int64_t)item * a.s_max;
-  const float* ml = a.ws_ml + base * 2;
-  const int cap = a.s_max < kMergeStage ? a.s_max : kMergeStage;
-  float* sm = stage + cap * 64;
-  float* sl = sm + cap;
-  // global max over all splits (every wave, lane-parallel)
-  float gm = -1e30f;
-  for (int s0 = 0; s0 < S; s0 += kWave) {
-    const float v = s0 + lane < S ? ml[(s0 + lane) * 2] : -1e30f;
-    gm = fmaxf(gm, wave_max(v));
-  }
-  float gl = 0.0f, out = 0.0f;
-  bool first = true;
-  for (int c0 = 0; c0 < S; c0 += kMergeStage) {
-    const int n = S - c0 < kMergeStage ? S - c0 : kMergeStage;
-    __syncthreads();
-    for (int r = wave; r < n; r += 4) stage[r * 64 + lane] = a.ws_acc[(base + c0 + r) * HD + col];
-    for (int r = threadIdx.x; r < n; r += 256) {
-      sm[r] = ml[(c0 + r) * 2];
-      sl[r] = ml[(c0 + r) * 2 + 1];
-    }
-    __syncthreads();
-    if (wave != 0) continue;
-    for (int s0 = 0; s0 < n; s0 += kWave) {
-      const int m = n - s0 < kWave ? n - s0 : kWave;
-      float d = -1e30f, ls = 0.0f;
-      if (lane < m) { d = sm[s0 + lane] - gm; ls = sl[s0 + lane]; }
-      float c = fast_exp_softmax_biased(max87(d));
-      if (!(ls > 0.0f)) c = 0.0f;
-      // global l: batches of 16 splits, each a 16-lane tree of l * c
-      const float bsum = tree16(ls * c);
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (16 * q < m) gl = gl + readlane_f(bsum, 16 * q);
-      const unsigned long long live = __ballot(lane < m && c > 0.0f);
-      const unsigned long long all = m == 64 ? ~0ull : ((1ull << m) - 1);
-      int b = 0;
-      if (first && (live & 1ull)) {  // the first contributing split is multiplied
-        out = stage[s0 * 64 + lane] * readlane_f(c, 0);
-        first = false;
-        b = 1;
-      }
-      if (!first && live == all) {
-        // every split contributes: branch-free chain, eight LDS rows per batch
-        for (; b + 8 <= m; b += 8) {
-          float v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) v[u] = stage[(s0 + b + u) * 64 + lane];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) out = fmaf(v[u], readlane_f(c, b + u), out);
-        }
-      }
-      for (; b < m; ++b) {
-        const float cb = readlane_f(c, b);
-        if (cb <= 0.0f) continue;
-        const float v = stage[(s0 + b) * 64 + lane];
-        out = first ? v * cb : fmaf(v, cb, out);
-        first = false;
-      }
-    }
-  }
-  if (wave != 0) return;
   uint16_t* dst = a.out + (int64_t)item * HD + col;
-  *dst = gl > 0.0f ? f32_to_bf16(out * (1.0f / gl)) : (uint16_t)0;
+#pragma unroll
+  for (int j = 0; j < CL; ++j) dst[j] = gl > 0.0f ? f32_to_bf16(out[j] * (1.0f / gl)) : (uint16_t)0;
 }
 
 // ---------------------------------------------------------------------------
@@ -868,39 +931,46 @@ hipError_t launch_attn_prep(const PrepArgs& args, int head_dim, hipStream_t st) 
 template <int HD>
 static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
   const dim3 b(256);
-  if (a.s_max == 1 && gqa <= 8 && HD <= 256) {
-    // one split per token: 16/G tokens per wave, finalized in the wave
-    const int tpw = 16 / gqa;
-    const int items = (a.T + 16 * tpw - 1) / (16 * tpw) * a.num_kv * 16;
-    const dim3 g((items + 3) / 4);
+  // Row groups need neighbours in a run to share tiles with: one-split plans
+  // (many tokens), and split plans with two groups' tokens per run (200 tokens
+  // of one run at position 2000, sliding: 178 -> 102 us).  A decode step's
+  // tokens share nothing: a wave each.
+  const int tpw = 16 / gqa, nblk = (a.T + 16 * tpw - 1) / (16 * tpw);
+  if (a.s_max == 1 || a.T >= 2 * tpw * a.num_runs) {
+    const int nh = attn_rows_lone(gqa, a.s_max) ? attn_rows_parts(gqa) : 1;
+    const dim3 g(nblk * 16 * nh * a.num_kv * a.s_max);
     switch (gqa) {
-      case 1: hipLaunchKernelGGL((k_flash_attn_mt<HD, 1>), g, b, 0, st, a); break;
-      case 2: hipLaunchKernelGGL((k_flash_attn_mt<HD, 2>), g, b, 0, st, a); break;
-      case 4: hipLaunchKernelGGL((k_flash_attn_mt<HD, 4>), g, b, 0, st, a); break;
-      case 8: hipLaunchKernelGGL((k_flash_attn_mt<HD, 8>), g, b, 0, st, a); break;
+      case 1: hipLaunchKernelGGL((k_flash_attn_rows<HD, 1>), g, b, 0, st, a, nblk); break;
+      case 2: hipLaunchKernelGGL((k_flash_attn_rows<HD, 2>), g, b, 0, st, a, nblk); break;
+      case 4: hipLaunchKernelGGL((k_flash_attn_rows<HD, 4>), g, b, 0, st, a, nblk); break;
+      case 8: hipLaunchKernelGGL((k_flash_attn_rows<HD, 8>), g, b, 0, st, a, nblk); break;
+      case 16: hipLaunchKernelGGL((k_flash_attn_rows<HD, 16>), g, b, 0, st, a, nblk); break;
       default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
-  }
-  const int items = a.T * a.num_kv * a.s_max;
-  const dim3 g((items + 3) / 4);
-  switch (gqa) {
-    case 1: hipLaunchKernelGGL((k_flash_attn<HD, 1>), g, b, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_flash_attn<HD, 2>), g, b, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_flash_attn<HD, 4>), g, b, 0, st, a); break;
-    case 8: hipLaunchKernelGGL((k_flash_attn<HD, 8>), g, b, 0, st, a); break;
-    case 16: hipLaunchKernelGGL((k_flash_attn<HD, 16>), g, b, 0, st, a); break;
-    default: return hipErrorInvalidValue;
+  } else {
+    const int items = a.T * a.num_kv * a.s_max;
+    const dim3 g((items + 3) / 4);
+    switch (gqa) {
+      case 1: hipLaunchKernelGGL((k_flash_attn<HD, 1>), g, b, 0, st, a); break;
+      case 2: hipLaunchKernelGGL((k_flash_attn<HD, 2>), g, b, 0, st, a); break;
+      case 4: hipLaunchKernelGGL((k_flash_attn<HD, 4>), g, b, 0, st, a); break;
+      case 8: hipLaunchKernelGGL((k_flash_attn<HD, 8>), g, b, 0, st, a); break;
+      case 16: hipLaunchKernelGGL((k_flash_attn<HD, 16>), g, b, 0, st, a); break;
+      default: return hipErrorInvalidValue;
+    }
   }
   if (a.s_max == 1) return hipGetLastError();  // every token finished in the wave
-  if (a.s_max > 8) {
-    const size_t lds = (size_t)(a.s_max < kMergeStage ? a.s_max : kMergeStage) * 66 * sizeof(float);
-    hipLaunchKernelGGL(k_attn_merge_lds<HD>, dim3(a.T * a.num_q * (HD / 64)), b, lds, st, a);
-  } else {
-    constexpr int NW = HD < 128 ? 1 : HD / 128;
-    const dim3 gm((a.T * a.num_q * NW + 3) / 4);
-    hipLaunchKernelGGL(k_attn_merge<HD>, gm, b, 0, st, a);
-  }
+  // up to 8 splits (many tokens): two columns per lane and as many rows in
+  // flight as the plan can have; more splits (few tokens): one column, 32 rows
+  // (64 splits, 16 tokens, head 512: 9.7 us; with the rows staged in LDS for one
+  // wave's chain 16.9)
+  constexpr int CL = HD >= 128 ? 2 : 1;
+  const int waves = a.T * a.num_q * (HD / 64);
+  const dim3 g2((waves / CL + 3) / 4), g1((waves + 3) / 4);
+  if (a.s_max <= 2) hipLaunchKernelGGL((k_attn_merge<HD, 2, CL>), g2, b, 0, st, a);
+  else if (a.s_max <= 4) hipLaunchKernelGGL((k_attn_merge<HD, 4, CL>), g2, b, 0, st, a);
+  else if (a.s_max <= 8) hipLaunchKernelGGL((k_attn_merge<HD, 8, CL>), g2, b, 0, st, a);
+  else hipLaunchKernelGGL((k_attn_merge<HD, 32, 1>), g1, b, 0, st, a);
   return hipGetLastError();
 }
 

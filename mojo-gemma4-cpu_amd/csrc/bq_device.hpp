@@ -124,6 +124,16 @@ __device__ inline float fast_exp_softmax_biased(float x) {
   return k * (QC_A + f * (QC_B + f * QC_C));
 }
 
+// fast_exp_softmax_biased for x in [-87, 0]: there v is in [6.3e6, 1.06e9],
+// so the truncation needs no range check; the same value.
+__device__ inline float fast_exp_softmax_le0(float x) {
+  const float v = 12102203.16156148f * x + 1059208216.0f;
+  const uint32_t u = (uint32_t)(int32_t)v;
+  const float f = (float)(u & 0x7FFFFFu) * (1.0f / (float)(1 << 23));
+  return __uint_as_float(u) * (1.6501418352127075f +
+                               f * (-0.37554836273193359f + f * 0.38696467876434326f));
+}
+
 // simd_math/ops.mojo:35-69 exp_f32: input clamped to [-87, 88] through
 // sign-bit masks, n = trunc(xn + 0.5 - sign(xn)), Cody-Waite reduction with
 // two ln2 constants, degree-6 polynomial, times 2^n.
@@ -187,6 +197,9 @@ __device__ inline float gumbel_noise(uint64_t seed, int64_t row, int64_t idx) {
 // wave helpers
 // ---------------------------------------------------------------------------
 __device__ inline int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
+
+template <int ST>
+struct Stride { static constexpr int value = ST; };
 
 // (after the cross-lane partner helpers below)
 template <int ST>
@@ -271,6 +284,43 @@ __device__ inline float row_shl(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x100 + H, 0xF, 0xF, false));
 }
 
+// v_max_f32 as it is: the larger, or the one that is a number (fmaxf would
+// first pass each operand through a canonicalizing v_max)
+__device__ inline float max_num(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// max over the 16 lanes of each row, in every lane of it, of four values at
+// once: DPP row rotations by 8, 4, 2, 1 (max takes any order; a NaN loses to a
+// number).  In asm: fmaxf would first pass each moved value through a
+// canonicalizing v_max.  Four values in turn keep two instructions between a
+// write and the DPP read of it.
+__device__ inline void row_max16_x4(float (&v)[4]) {
+#define BQ_ROR(n)                                                  \
+  "v_max_f32_dpp %0, %0, %0 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_max_f32_dpp %1, %1, %1 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_max_f32_dpp %2, %2, %2 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_max_f32_dpp %3, %3, %3 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t" BQ_ROR(8) BQ_ROR(4) BQ_ROR(2) BQ_ROR(1) "s_nop 0"
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#undef BQ_ROR
+}
+
+// the tree16 of the attention's 16-position tiles, in lane 0 of each row of 16
+// lanes (the other lanes hold values of no use)
+__device__ inline float row_tree16(float v) {
+  auto add = [](float x, auto n) {
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x100 + decltype(n)::value,
+                                                       0xF, 0xF, true));  // row_shl, 0 past the row
+  };
+  v = add(v, Stride<8>{});
+  v = add(v, Stride<4>{});
+  v = add(v, Stride<2>{});
+  return add(v, Stride<1>{});
+}
+
 // One element of a cross-lane FWHT stage of stride ST: the lane with bit ST
 // clear holds a and gets a + b, its partner holds b and gets a - b.  Computed
 // as fmaf(s, v, p) with s = +1 / -1 and p the partner's value: s*v is exact,
@@ -279,9 +329,6 @@ template <int ST>
 __device__ inline float xlane_bfly(float v) {
   return fmaf((threadIdx.x & ST) ? -1.0f : 1.0f, v, xlane_partner<ST>(v));
 }
-
-template <int ST>
-struct Stride { static constexpr int value = ST; };
 
 // f(Stride<ST>{}) for the cross-lane strides ST = 1, 2, 4, ... below
 // min(block, 64), in that order.
@@ -423,6 +470,23 @@ __device__ inline v4i mfma16x16x64(v4i a, v4i b, v4i c) {
 // POPS with 16 independent chains per wave; this one ~4.8 with 4).
 __device__ inline v16i mfma32x32x32(v4i a, v4i b, v16i c) {
   return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+}
+
+// f32, 16x16 output, 4 of K: A lane L = row L%16, k = L/16; B lane L = column
+// L%16, k = L/16; D lane L register i = row 4*(L/16) + i, column L%16.  The
+// four products are added as fmaf in k order, each rounded once, denormals
+// kept: bit for bit a chain of four fmaf (checked against it over normal,
+// denormal and mixed inputs).
+typedef float v4f __attribute__((ext_vector_type(4)));
+__device__ inline v4f mfma16x16x4f(float a, float b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// f32, sixteen blocks of 4x4 output, 1 of K; with the same four rows in every
+// block a 4x64 output: A lane L = row L%4, B lane L = column L, D lane L
+// register i = row i, column L.  One fmaf per output, as above.
+__device__ inline v4f mfma4x64x1f(float a, float b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave by DPP adds: row_shr 1,

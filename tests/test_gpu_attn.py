@@ -185,3 +185,31 @@ def test_prep_then_attention(gpu, O):
     ref = O.flash_attention(rqi, rqb, rfq, p["kc"], p["ks"], p["vc"], p["vs"], p["runs"],
                             p["rows"], nq, nkv, hd, 48, p["shift"], page - 1, -1, s_max=s_max)
     np.testing.assert_array_equal(host(out), ref)
+
+
+@pytest.mark.parametrize("gqa,hd", [(1, 64), (2, 128), (2, 256), (4, 128), (8, 512), (16, 64)])
+@pytest.mark.parametrize("window,seqs,s_max", [
+    (0, [(0, 75)], 2),               # neighbours in small sets; a ragged last block
+    (0, [(200, 40), (3, 17)], 5),    # two runs in one block, starts unequal mod 16
+    (40, [(90, 49)], 2),             # every window slides: tokens 16 apart
+    (40, [(20, 37), (0, 64)], 3),    # windows start to slide inside a run; a run that begins at 0
+    (33, [(31, 33)], 1),             # lengths of one position past two tiles
+])
+def test_attention_row_groups_split(gpu, O, gqa, hd, window, seqs, s_max):
+    # chunks of many tokens per run: 16 / gqa tokens share a workgroup, those
+    # with equal tile grids a set; more splits than some tokens have positions for
+    c = make_case(O, gqa * 5 + hd + window, num_q=gqa, num_kv=1, head_dim=hd, page_len=32,
+                  window=window, ring_pages=4, seqs=seqs)
+    check(gpu, O, c, s_max)
+
+
+def test_attention_row_groups_extremes(gpu, O):
+    # zero scales, infinite scores and scores far below the running maximum
+    c = make_case(O, 77, num_q=4, num_kv=2, head_dim=128, page_len=64, window=48, ring_pages=4,
+                  seqs=[(70, 66), (0, 35)])
+    c.k_scale[::7] = 0.0
+    c.k_scale[3::11] *= 1e4
+    c.v_scale[::5] = 1e-38
+    c.f_q[::9] *= 1e30
+    for s_max in (1, 2):
+        check(gpu, O, c, s_max)

@@ -231,6 +231,162 @@ __global__ __launch_bounds__(256) void k_attn_prep(PrepArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Attention prep of many tokens: four heads of one token per wave, eight
+// consecutive values per lane (head_dim / 8 lanes a head, so 512 / head_dim
+// heads per round).  k_attn_prep is bound by vector-ALU issue and by its one-
+// and two-byte accesses; here rows are 16-byte loads and 8-byte stores, the
+// FWHT's strides 1, 2, 4 stay inside the lane, and the four heads' sums of
+// squares (lane k + 16 h: chain k of head h, from LDS), square roots and
+// divisions share their instructions.  Takes pair_stride == head_dim / 2, 16-
+// byte aligned sources, gains and tables and 8-byte aligned codes.  The same
+// values in the same order as k_attn_prep, to the bit: in the cross-lane
+// stages within a row the upper lane of a pair holds -(a - b), and the sign
+// (the parity of its index bits) is folded into the final scale, as in
+// nq_v8_transform.
+// ---------------------------------------------------------------------------
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_prep_v8(PrepArgs a) {
+  constexpr int LPH = HD / 8, HPR = kWave / LPH, RND = 4 / HPR;  // lanes a head; heads a round; rounds
+  static_assert(HPR >= 1 && RND >= 1, "128 <= head_dim <= 512");
+  // (16 values of padding: the four heads' chains read different banks)
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[4][4][HD + 16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+  const int nh = a.num_q + 2 * a.num_kv, hg = (nh + 3) / 4;  // a token's waves
+  const int item = blockIdx.x * 4 + wave, tok = item / hg, j0 = (item % hg) * 4;
+  if (tok >= a.T) return;
+  const int r = run_of(a.runs, a.num_runs, tok);
+  const KvRun run = a.runs[r];
+  const int64_t pos = (int64_t)run.base_pos + (tok - run.buf_start);
+  const int64_t kvs = (int64_t)a.num_kv * HD;
+  const int sub = lane / LPH;  // head within the round
+  const int run8 = dpp_run(lane % LPH), e0 = run8 * 8;  // this lane's values of it
+  v4i raw[RND];
+#pragma unroll
+  for (int q = 0; q < RND; ++q) {
+    const int j = min(j0 + q * HPR + sub, nh - 1);  // (heads past the last: read, never stored)
+    const uint16_t* src = j < a.num_q ? a.q_src + (int64_t)tok * a.num_q * HD + j * HD
+                          : j < a.num_q + a.num_kv
+                              ? a.k_src + tok * kvs + (j - a.num_q) * HD
+                              : a.v_src + tok * kvs + (j - a.num_q - a.num_kv) * HD;
+    raw[q] = *reinterpret_cast<const v4i*>(src + e0);
+    *reinterpret_cast<v4i*>(&s_x[wave][q * HPR + sub][e0]) = raw[q];
+  }
+  // The position's rotation.  A pair's halves are LPH / 2 lanes apart (a row or
+  // more), and go through exchanged pairs of values (row_exchange): value pair
+  // i, i + 1 leaves value i + up here, so this lane needs every other entry.
+  const int up = (lane / (LPH / 2)) & 1;
+  const int el = (run8 % (LPH / 2)) * 8;
+  const bool rot = el < a.rope_half;
+  float cs[4], sn[4];
+  if constexpr (LPH >= 32) {
+    const int64_t o = pos * a.rope_half + (rot ? el : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      cs[i] = a.cos_table[o + 2 * i + up];
+      sn[i] = a.sin_table[o + 2 * i + up];
+    }
+  }
+  // head_inv_rms: chain lane & 15 of head j0 + lane / 16, then the 16-lane tree
+  float ssq;
+  {
+    const uint16_t* x = &s_x[wave][lane >> 4][lane & 15];
+    const float x0 = bf16_to_f32(x[0]);
+    ssq = x0 * x0;
+#pragma unroll
+    for (int i = 1; i < HD / 16; ++i) {
+      const float xi = bf16_to_f32(x[16 * i]);
+      ssq = fmaf(xi, xi, ssq);
+    }
+    ssq = row_tree16(ssq);
+  }
+  const float inv4 = a.sqrt_n / __builtin_sqrtf(ssq + a.n_eps);  // lane 16 h: head h's
+  const float scale = (__builtin_popcount(run8 & 15) & 1) ? -a.fwht_scale : a.fwht_scale;
+  const float s1 = run8 & 1 ? -1.0f : 1.0f, s2 = run8 & 2 ? -1.0f : 1.0f;
+  const float s4 = run8 & 4 ? -1.0f : 1.0f, s8 = run8 & 8 ? -1.0f : 1.0f;
+  // attention.mojo:515: K/V rows (and pages) only for positions this cache rank owns
+  const bool owned = pos % a.cache_degree == a.rank;
+  const int64_t slot = owned ? paged_slot(a.base_rows + run.rows_off, a.page_shift, a.row_mask,
+                                          a.page_mask, pos / a.cache_degree) : 0;
+#pragma unroll
+  for (int q = 0; q < RND; ++q) {
+    const int j = j0 + q * HPR + sub;
+    const bool is_q = j < a.num_q, is_v = j >= a.num_q + a.num_kv;
+    const float inv = __shfl(inv4, 16 * (q * HPR + sub), kWave);
+    float v[8], g[8];
+    bf16x8_to_f32(raw[q], v);
+    v4i gr = *reinterpret_cast<const v4i*>((is_q ? a.q_norm : a.k_norm) + e0);
+    if (is_v) gr = v4i{0x3F803F80, 0x3F803F80, 0x3F803F80, 0x3F803F80};  // no gain: times 1
+    bf16x8_to_f32(gr, g);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * g[i];
+    if constexpr (LPH >= 32) {
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        float lo, hi;
+        row_exchange<LPH / 2>(v[i], v[i + 1], lo, hi);
+        const float c = cs[i / 2], s = sn[i / 2];
+        const float nl = lo * c - hi * s, nu = hi * c + lo * s;
+        row_exchange<LPH / 2>(rot && !is_v ? nl : lo, rot && !is_v ? nu : hi, v[i], v[i + 1]);
+      }
+    } else {
+      const int64_t o = pos * a.rope_half + (rot ? el : 0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float c = a.cos_table[o + i], s = up ? a.sin_table[o + i] : -a.sin_table[o + i];
+        const float n = v[i] * c + xlane_partner<LPH / 2>(v[i]) * s;
+        v[i] = rot && !is_v ? n : v[i];
+      }
+    }
+#pragma unroll
+    for (int st = 1; st < 8; st <<= 1)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i & st) continue;
+        const float x = v[i], y = v[i + st];
+        v[i] = x + y;
+        v[i + st] = x - y;
+      }
+    dpp_bfly8<1>(v, s1);
+    dpp_bfly8<2>(v, s2);
+    dpp_bfly8<4>(v, s4);
+    dpp_bfly8<8>(v, s8);
+    if constexpr (LPH >= 32) row_bfly8<16>(v);
+    if constexpr (LPH >= 64) row_bfly8<32>(v);
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = v[i] * scale;
+      amax = fmaxf(amax, fabsf(v[i]));
+    }
+    for_each_xlane_stride(LPH, [&](auto st) {
+      amax = fmaxf(amax, xlane_partner<decltype(st)::value>(amax));
+    });
+    if (amax < 1e-10f) amax = 1e-10f;
+    uint32_t w[2];
+    codes8_bounded(v, 127.0f / amax, w);  // (amax >= 1e-10: a finite factor)
+    int qs = __builtin_amdgcn_sdot4((int)w[1], 0x01010101,
+                                    __builtin_amdgcn_sdot4((int)w[0], 0x01010101, 0, false), false);
+    for_each_xlane_stride(LPH, [&](auto st) {  // the head's code sum
+      qs += __float_as_int(xlane_partner<decltype(st)::value>(__int_as_float(qs)));
+    });
+    if (j >= nh || (!is_q && !owned)) continue;
+    const int h = is_q ? j : is_v ? j - a.num_q - a.num_kv : j - a.num_q;
+    int8_t* dst = is_q ? a.q_i8 + ((int64_t)tok * a.num_q + h) * HD
+                       : (is_v ? a.v_cache : a.k_cache) + slot * kvs + (int64_t)h * HD;
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    *reinterpret_cast<u2*>(dst + e0) = u2{w[0], w[1]};
+    if (e0 == 0) {
+      if (is_q) {
+        a.qi_bias[(int64_t)tok * a.num_q + h] = (float)qs * 128.0f;
+        a.f_q[(int64_t)tok * a.num_q + h] = amax;
+      } else {
+        (is_v ? a.v_scale : a.k_scale)[slot * a.num_kv + h] = amax;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // flash attention: one wave per (token, kv head, split); G query heads share
 // the kv head (G <= 16).  wsh: the wave's LDS for 16 x G weights [p][head].
 // ---------------------------------------------------------------------------
@@ -912,12 +1068,32 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// (token, head) items from which the prep takes four heads per wave: 3200 items
+// (100 tokens, 32 heads of 256) 1.3 us faster than a wave per head, 65536 items
+// 48.4 -> 23.4 us; below 2048 a wave per item still leaves CUs to spare
+constexpr int kPrepV8Items = 2048;
+
 hipError_t launch_attn_prep(const PrepArgs& args, int head_dim, hipStream_t st) {
   PrepArgs a = args;
   a.fwht_scale = fwht_scale_host(head_dim);
   const int items = a.T * (a.num_q + 2 * a.num_kv);
   if (items <= 0) return hipSuccess;
   const dim3 g((items + 3) / 4), b(256);
+  auto aligned = [](const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; };
+  if (head_dim >= 128 && items >= kPrepV8Items && a.pair_stride == head_dim / 2 &&
+      a.rope_half > 0 && aligned(a.q_src, 16) && aligned(a.k_src, 16) &&
+      aligned(a.v_src, 16) && aligned(a.q_norm, 16) && aligned(a.k_norm, 16) &&
+      aligned(a.cos_table, 16) && aligned(a.sin_table, 16) && aligned(a.q_i8, 8) &&
+      aligned(a.k_cache, 8) && aligned(a.v_cache, 8)) {
+    const dim3 gv((a.T * ((a.num_q + 2 * a.num_kv + 3) / 4) + 3) / 4);
+    switch (head_dim) {
+      case 128: hipLaunchKernelGGL(k_attn_prep_v8<128>, gv, b, 0, st, a); break;
+      case 256: hipLaunchKernelGGL(k_attn_prep_v8<256>, gv, b, 0, st, a); break;
+      case 512: hipLaunchKernelGGL(k_attn_prep_v8<512>, gv, b, 0, st, a); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   switch (head_dim) {
     case 64: hipLaunchKernelGGL(k_attn_prep<1>, g, b, 0, st, a); break;
     case 128: hipLaunchKernelGGL(k_attn_prep<2>, g, b, 0, st, a); break;

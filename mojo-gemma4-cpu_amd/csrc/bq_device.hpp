@@ -734,6 +734,84 @@ __device__ inline void nq_v8_codes(const float (&v)[8], float inv, uint32_t (&w)
     w[j >> 2] |= (uint32_t)(uint8_t)quantize_i8(v[j], inv) << (8 * (j & 3));
 }
 
+// ---------------------------------------------------------------------------
+// One-instruction butterflies of 8 values per lane.  v + s * partner with the
+// partner read by DPP inside the fma: strides 1, 2, 8 as quad permutations and
+// a rotation by 8; DPP has no exchange of lanes 4 apart, but mirrors half rows
+// (lane ^ 7), so index bit 2 is laid out as that: lane L holds run
+// dpp_run(L) = L ^ 3 where bit 2 of L is set, and s = -1 where dpp_run's bit
+// is set.  Eight values in turn keep every write eight instructions from the
+// DPP read of it.
+__device__ inline int dpp_run(int lane) { return lane & 4 ? lane ^ 3 : lane; }
+
+template <int ST>
+__device__ inline void dpp_bfly8(float (&v)[8], float s) {
+#define BQ_BFLY(ctrl)                                                                           \
+  asm("s_nop 1\n\t"                                                                            \
+      "v_fmac_f32_dpp %0, %0, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %1, %1, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %2, %2, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %3, %3, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %4, %4, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %5, %5, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %6, %6, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f32_dpp %7, %7, %8 " ctrl " row_mask:0xf bank_mask:0xf"                           \
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]),     \
+        "+v"(v[7])                                                                              \
+      : "v"(s))
+  if constexpr (ST == 1) BQ_BFLY("quad_perm:[1,0,3,2]");
+  else if constexpr (ST == 2) BQ_BFLY("quad_perm:[2,3,0,1]");
+  else if constexpr (ST == 4) BQ_BFLY("row_half_mirror");
+  else BQ_BFLY("row_ror:8");
+#undef BQ_BFLY
+}
+
+// Rows r and r ^ ST/16 (ST 16 or 32) of a pair of values: lo holds the lower
+// rows' x (in the lower rows) and y (in the upper), hi the upper rows'; the
+// same exchange of (lo, hi) brings them back.
+template <int ST>
+__device__ inline void row_exchange(float x, float y, float& lo, float& hi) {
+  const unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+  if constexpr (ST == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+  }
+}
+
+// a butterfly stage of lane stride 16 or 32 on 8 values per lane: a + b in the
+// lower rows, a - b in the upper, a pair of values per exchange
+template <int ST>
+__device__ inline void row_bfly8(float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    float lo, hi;
+    row_exchange<ST>(v[i], v[i + 1], lo, hi);
+    row_exchange<ST>(lo + hi, lo - hi, v[i], v[i + 1]);
+  }
+}
+
+// the codes of 8 values with |v * inv| <= 127.5 or NaN (code 0): adding 1.5 *
+// 2^23 rounds half to even and leaves the code in the low byte
+__device__ inline void codes8_bounded(const float (&v)[8], float inv, uint32_t (&w)[2]) {
+  uint32_t u[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float t = v[i] * inv;
+    u[i] = __float_as_uint(t + 12582912.0f);
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t p0 = __builtin_amdgcn_perm(u[4 * h + 1], u[4 * h], 0x0C0C0400u);
+    const uint32_t p1 = __builtin_amdgcn_perm(u[4 * h + 3], u[4 * h + 2], 0x04000C0Cu);
+    w[h] = p0 | p1;
+  }
+}
+
 // the int8 code pair of v[i] (low byte: the even element)
 __device__ inline uint16_t nq_pair_code(const float (&vi)[2], float inv) {
   return (uint16_t)((uint8_t)quantize_i8(vi[0], inv) | ((uint16_t)(uint8_t)quantize_i8(vi[1], inv) << 8));

@@ -213,3 +213,31 @@ def test_attention_row_groups_extremes(gpu, O):
     c.f_q[::9] *= 1e30
     for s_max in (1, 2):
         check(gpu, O, c, s_max)
+
+
+@pytest.mark.parametrize("hd,rope_half,nq,nkv,degree,rank,ntok", [
+    (256, 128, 16, 8, 1, 0, 64),    # four waves of four heads, twice a token; the fewest tokens
+    (512, 64, 16, 2, 2, 1, 116),    # a last wave of a token alone; cache rank 1 of 2
+    (128, 64, 13, 3, 1, 0, 131),    # heads past the token's last
+    (256, 64, 6, 5, 3, 0, 140),     # waves that mix q, k and v heads
+    (256, 0, 16, 8, 1, 0, 64),      # no RoPE: one head per wave
+])
+def test_attn_prep_many_tokens(gpu, O, hd, rope_half, nq, nkv, degree, rank, ntok):
+    # enough (token, head) items for four heads per wave
+    import torch
+    p = prep_case(O, hd + nq + 1, hd, rope_half, hd // 2, nq, nkv, [(100, ntok - 21), (3, 21)], 64,
+                  degree, rank)
+    p["q"][5, :hd] = 0  # a head of zeros: the smallest scale
+    g = {n: dev(p[n]) for n in ("kc", "ks", "vc", "vs")}
+    runs = dev(np.ascontiguousarray(p["runs"]).view(np.int32).reshape(-1, 4))
+    args = (nq, nkv, hd, rope_half, hd // 2, p["shift"], p["page"] - 1, -1)
+    got = gpu.attn_prep(dev(p["q"]), dev(p["k"]), dev(p["v"]), dev(p["qn"]), dev(p["kn"]), g["kc"],
+                        g["ks"], g["vc"], g["vs"], dev(p["cos"]), dev(p["sin"]), runs,
+                        dev(p["rows"]), *args, cache_degree=degree, rank=rank)
+    torch.cuda.synchronize()
+    ref = O.attn_prep(p["q"], p["k"], p["v"], p["qn"], p["kn"], p["kc"], p["ks"], p["vc"], p["vs"],
+                      p["cos"], p["sin"], p["runs"], p["rows"], *args, cache_degree=degree, rank=rank)
+    for x, y in zip(got, ref):
+        np.testing.assert_array_equal(host(x).view(np.uint8), y.view(np.uint8))
+    for n in ("kc", "ks", "vc", "vs"):
+        np.testing.assert_array_equal(host(g[n]).view(np.uint8), p[n].view(np.uint8))

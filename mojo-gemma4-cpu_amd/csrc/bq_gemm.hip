@@ -427,6 +427,40 @@ void k_gemv_m1_1(BQ_SEG1_PARAMS) {
 // ---------------------------------------------------------------------------
 // launcher
 // ---------------------------------------------------------------------------
+// The tile of a linear of more than 32 rows: the one whose rounds of
+// workgroups over the CUs take least.  A larger tile reads fewer operand bytes
+// per product (the k loop is bound by the CU's intake from L2, 21-24 B/clk),
+// but a last round that is nearly empty costs as much as a full one.  `cost`
+// is a round's time in us per 1000 of K, measured (per-row: 2048 x 8192 at K =
+// 2816 four rounds of 128 x 128 79 us, one of 256 x 256 50; 1111 x 9216 three
+// of 128 x 128 58, one of 192 x 256 39; 512 x 4096 at K = 4096 one of 64 x 128
+// 14, 128 x 256 36.  Per-block: 2048 x 2816 at K = 4096 two rounds of 128 x
+// 128 74, one of 192 x 128 50; 1111 x 2816 at K = 8192 396 of 64 x 128, two to
+// a CU, 75, 198 of 128 x 128 66).
+static void pick_linear_tile(const LinArgs& a, int per_block, int& bm, int& bn) {
+  struct Tile { int bm, bn; float cost; };
+  static const Tile row[] = {{64, 128, 3.5f}, {128, 128, 6.5f}, {192, 128, 9.6f},
+                             {128, 256, 11.5f}, {192, 256, 14.0f}, {256, 256, 17.6f}};
+  static const Tile blk[] = {{64, 128, 5.5f}, {128, 128, 8.6f}, {192, 128, 11.5f}, {128, 256, 13.5f}};
+  const Tile* t = per_block ? blk : row;
+  const int nt = per_block ? 4 : 6;
+  float best = 0.0f;
+  for (int i = 0; i < nt; ++i) {
+    int gn = 0;
+    for (int q = 0; q < a.nseg; ++q) gn += (a.seg[q].n + t[i].bn - 1) / t[i].bn;
+    const int tiles = (a.M + t[i].bm - 1) / t[i].bm * gn;
+    float rounds = (float)((tiles + tune().cus - 1) / tune().cus);
+    // (64 x 128 per-block tiles run two to a CU, at 9.1 the pair)
+    if (per_block && t[i].bm == 64 && rounds > 1.0f)
+      rounds = (float)((tiles + 2 * tune().cus - 1) / (2 * tune().cus)) * (9.1f / 5.5f);
+    if (i > 0 && (rounds * t[i].cost >= best || !linear_tile_fits(a, per_block, t[i].bm, t[i].bn)))
+      continue;
+    best = rounds * t[i].cost;
+    bm = t[i].bm;
+    bn = t[i].bn;
+  }
+}
+
 hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
   if (a.M <= 0) return hipSuccess;
   if (a.M <= 16) {
@@ -493,14 +527,11 @@ hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
 #undef BQ_GO
     return hipGetLastError();
   }
-  // prefer the largest M tile that still yields >= 256 workgroups (one per CU)
-  int gn128 = 0;
-  for (int q = 0; q < a.nseg; ++q) gn128 += (a.seg[q].n + 127) / 128;
-  int bm = 32;
-  if (a.M > 64 && ((a.M + 127) / 128) * gn128 >= 256) bm = 128;
-  else if (a.M > 32) bm = 64;
+  int bm = 32, bn = 128;
+  if (a.M > 32) pick_linear_tile(a, per_block, bm, bn);
   if (tune().tile_bm) bm = tune().tile_bm;
-  return launch_linear_tiled(a, per_block, bm, st);
+  if (tune().tile_bn) bn = tune().tile_bn;
+  return launch_linear_tiled(a, per_block, bm, bn, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -16,7 +16,7 @@ struct Tune {
   int gemv_waves;   // BQ_GEMV_WAVES: waves per workgroup of the general M <= 16 kernel (4, 8, 16;
                    // default 16); set, it also takes M = 1 per-row from k_gemv_m1
   int gemv_m1_waves;  // BQ_GEMV_M1_WAVES: waves per k_gemv_m1 workgroup (2, 4, 8)
-  int tile_bm;      // BQ_TILE_BM: rows per tiled prefill tile (32, 64, 128)
+  int tile_bm;      // BQ_TILE_BM: rows per tiled prefill tile (32, 64, 128, 192, 256)
   int tile_bn;      // BQ_TILE_BN: columns per tiled tile (128, 256)
   int ring;         // BQ_RING: LDS ring stages of the tiled kernels
   int tile_ksp;     // BQ_TILE_KSP: K groups per 64 x 128 prefill tile (1, 2)
@@ -98,7 +98,9 @@ hipError_t launch_norm_linear(const LinArgs& a, const NormArgs& nq, hipStream_t 
 
 struct Route { int32_t token; float weight; };
 
-hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, hipStream_t st);
+hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, int bn, hipStream_t st);
+// whether a bm x bn tile's operand ring and block scales fit in LDS
+bool linear_tile_fits(const LinArgs& a, int per_block, int bm, int bn);
 hipError_t launch_moe_gate_up_tiled(const int8_t* x_i8, const float* x_sa, const int32_t* eo,
                                     const Route* routes, const int8_t* w_gu, const float* gu_scale,
                                     uint16_t* bucket, int8_t* bi8, float* bsa, int experts,

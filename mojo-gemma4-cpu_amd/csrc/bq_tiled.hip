@@ -904,14 +904,20 @@ static void launch_bm(int bm, int bn, int nbuf, dim3 g, size_t dyn, hipStream_t 
 
 static inline int tile_bn(int bn) { return bn >= 256 ? 256 : 128; }
 
-hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, hipStream_t st) {
-  const int bn = tile_bn(or_default(tune().tile_bn, 128));
+bool linear_tile_fits(const LinArgs& a, int per_block, int bm, int bn) {
+  const size_t dyn = per_block ? (size_t)bm * (a.K / a.block) * sizeof(float) : 0;
+  return 2 * (size_t)(bm + bn) * 128 + dyn <= kLdsBytes;
+}
+
+hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, int bn, hipStream_t st) {
+  const int bmv = bm >= 256 ? 256 : bm >= 192 ? 192 : bm >= 128 ? 128 : bm >= 64 ? 64 : 32;
+  // (per-block tiles of 192 or 256 rows are 128 columns wide: launch_bm_mf)
+  bn = per_block && bmv >= 192 ? 128 : tile_bn(bn);
   const int nbuf = or_default(tune().ring, 3);
   TiledArgs t{};
   t.lin = a;
   int gn = 0;
   for (int q = 0; q < a.nseg; ++q) gn += (a.seg[q].n + bn - 1) / bn;
-  const int bmv = bm >= 128 ? 128 : bm >= 64 ? 64 : 32;
   t.gm = (a.M + bmv - 1) / bmv;
   t.gn = gn;
   dim3 g(t.gm * t.gn);
@@ -930,8 +936,7 @@ hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, hipStrea
     try_launch<MODE_DENSE, 64, 128, 2, 4, false, 2, 2>(g, 0, st, t);
     return hipGetLastError();
   }
-  // the grid is sized for bmv-row tiles, so the tile height is bmv (a larger
-  // BQ_TILE_BM is clamped to it)
+  // the grid is sized for bmv x bn tiles, the instances' own
   if (per_block) launch_bm<MODE_DENSE, true>(bmv, bn, nbuf, g, dyn, st, t);
   else launch_bm<MODE_DENSE, false>(bmv, bn, nbuf, g, dyn, st, t);
   return hipGetLastError();

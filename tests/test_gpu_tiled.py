@@ -38,6 +38,14 @@ def test_dense_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B):
     np.testing.assert_array_equal(host(ob), rb)
 
 
+@pytest.mark.parametrize("bm,bn", [(192, 128), (192, 256), (256, 256)])
+@pytest.mark.parametrize("M,K,B", [(193, 704, None), (511, 320, None), (255, 1024, 256), (400, 2112, 64)])
+def test_dense_tall_tiles(gpu, O, tune_env, bm, bn, M, K, B):
+    # the taller tiles of large chunks: a last tile of one row, of all but one,
+    # odd k-steps, and 1.5 n-tiles
+    test_dense_tiles(gpu, O, tune_env, bm, bn, 16, M, K, B)
+
+
 @pytest.mark.parametrize("mf", [16, 32])
 @pytest.mark.parametrize("M,K,N", [(200, 512, 384), (77, 2816, 384), (512, 4096, 4096),
                                    (64, 128, 256), (130, 704, 256), (33, 192, 128)])

@@ -614,11 +614,15 @@ static inline int mtile_bound(int max_routes, int experts, int bm) {
 // tiled tiles once each expert's weights can be reused.  The tile is sized
 // so that nearly every expert fits in one m-tile (mean + 4 standard
 // deviations of a binomial count): then each expert's weights stream from
-// HBM once instead of once per m-tile.
+// HBM once instead of once per m-tile.  From 15 routes per expert most experts
+// would fill two 16-row tiles and stream their weights twice (top-8 of 128,
+// the expert block in 16 / 64-row tiles: 200 tokens 168 / 172 us, 256 tokens
+// 209 / 174, 333 tokens 254 / 181; 100 tokens of 64 experts 95 / 97, 160 138 /
+// 103; with the dense MLP 200 tokens 224 / 244, 256 286 / 264).
 int moe_tile_bm(int max_routes, int experts) {
   if (tune().moe_bm) return tune().moe_bm;
   const int per = max_routes / (experts > 0 ? experts : 1);
-  if (per < 24) return 16;
+  if (per < 15) return 16;
   const double hi = per + 4.0 * __builtin_sqrt((double)per);
   if (hi > 192.0) return 256;
   if (hi > 128.0) return 192;  // 2048 tokens x top-8 / 128 experts: 128 + 45

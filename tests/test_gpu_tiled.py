@@ -39,7 +39,7 @@ def test_dense_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B):
 
 
 @pytest.mark.parametrize("bm,bn", [(192, 128), (192, 256), (256, 256)])
-@pytest.mark.parametrize("M,K,B", [(193, 704, None), (511, 320, None), (255, 1024, 256), (400, 2112, 64)])
+@pytest.mark.parametrize("M,K,B", [(193, 640, None), (511, 384, None), (255, 1024, 256), (400, 2112, 64)])
 def test_dense_tall_tiles(gpu, O, tune_env, bm, bn, M, K, B):
     # the taller tiles of large chunks: a last tile of one row, of all but one,
     # odd k-steps, and 1.5 n-tiles

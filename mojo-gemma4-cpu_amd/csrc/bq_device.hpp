@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace bq {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -193,6 +195,15 @@ __device__ inline float gumbel_noise(uint64_t seed, int64_t row, int64_t idx) {
   return -log_f32(-log_f32(u));
 }
 
+// f(std::integral_constant<int, I>{}) for I = I0 .. I1 - 1, in order
+template <int I0, int I1, typename F>
+__device__ inline void static_for(F&& f) {
+  if constexpr (I0 < I1) {
+    f(std::integral_constant<int, I0>{});
+    static_for<I0 + 1, I1>(f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // wave helpers
 // ---------------------------------------------------------------------------
@@ -308,17 +319,16 @@ __device__ inline void row_max16_x4(float (&v)[4]) {
 #undef BQ_ROR
 }
 
+// v + the value H lanes up in its row of 16 lanes (+ 0 past the row's end)
+template <int H>
+__device__ inline float row_add_shl(float v) {
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x100 + H, 0xF, 0xF, true));
+}
+
 // the tree16 of the attention's 16-position tiles, in lane 0 of each row of 16
 // lanes (the other lanes hold values of no use)
 __device__ inline float row_tree16(float v) {
-  auto add = [](float x, auto n) {
-    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x100 + decltype(n)::value,
-                                                       0xF, 0xF, true));  // row_shl, 0 past the row
-  };
-  v = add(v, Stride<8>{});
-  v = add(v, Stride<4>{});
-  v = add(v, Stride<2>{});
-  return add(v, Stride<1>{});
+  return row_add_shl<1>(row_add_shl<2>(row_add_shl<4>(row_add_shl<8>(v))));
 }
 
 // One element of a cross-lane FWHT stage of stride ST: the lane with bit ST
@@ -438,13 +448,25 @@ __device__ inline float wave_row_ssq(const uint32_t* __restrict__ pairs, int hid
   const int iters = hidden / (pu * 32);
   const int c0 = min(lane, chains - 1), c1 = min(lane + 64, chains - 1);
   float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll 4
-  for (int i = 0; i < iters; ++i) {
-    const uint32_t p0 = pairs[i * chains + c0], p1 = pairs[i * chains + c1];
-    a0 = fmaf(__uint_as_float(p0 & 0xFFFF0000u), __uint_as_float(p0 & 0xFFFF0000u), a0);
-    a0 = fmaf(__uint_as_float(p0 << 16), __uint_as_float(p0 << 16), a0);
-    a1 = fmaf(__uint_as_float(p1 & 0xFFFF0000u), __uint_as_float(p1 & 0xFFFF0000u), a1);
-    a1 = fmaf(__uint_as_float(p1 << 16), __uint_as_float(p1 << 16), a1);
+  // a batch's pairs are all requested before its chain runs (one memory round
+  // trip for rows of up to 3072 values)
+  constexpr int NB = 12;
+  for (int i0 = 0; i0 < iters; i0 += NB) {
+    uint32_t p0[NB], p1[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int i = min(i0 + b, iters - 1);
+      p0[b] = pairs[i * chains + c0];
+      p1[b] = pairs[i * chains + c1];
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (i0 + b >= iters) break;
+      a0 = fmaf(__uint_as_float(p0[b] & 0xFFFF0000u), __uint_as_float(p0[b] & 0xFFFF0000u), a0);
+      a0 = fmaf(__uint_as_float(p0[b] << 16), __uint_as_float(p0[b] << 16), a0);
+      a1 = fmaf(__uint_as_float(p1[b] & 0xFFFF0000u), __uint_as_float(p1[b] & 0xFFFF0000u), a1);
+      a1 = fmaf(__uint_as_float(p1[b] << 16), __uint_as_float(p1[b] << 16), a1);
+    }
   }
   float sum = 0.0f;
 #pragma unroll

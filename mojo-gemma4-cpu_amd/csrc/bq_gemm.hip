@@ -324,15 +324,6 @@ __global__ __launch_bounds__(1024) void k_linear_skinny2(LinArgs args) {
 // ---------------------------------------------------------------------------
 // M = 1, per-row (the decode GEMV)
 // ---------------------------------------------------------------------------
-// f(std::integral_constant<int, I>{}) for I = I0 .. I1 - 1, in order
-template <int I0, int I1, typename F>
-__device__ inline void static_for(F&& f) {
-  if constexpr (I0 < I1) {
-    f(std::integral_constant<int, I0>{});
-    static_for<I0 + 1, I1>(f);
-  }
-}
-
 // the four dwords of x as lane (lane + R) of the same 16-lane row holds them
 // (DPP row_shl:R); R = 0 is x itself
 template <int R>

@@ -30,7 +30,11 @@ constexpr float kRouterSentinel = -1.0e30f;
 // CPL adjacent chains c = l*CPL + r of the PU = CPL*4 accumulator bank
 // (64*CPL chains); per step i it scales its TT x values on the fly
 // ((x * router_scale) * inv_rms, :177-181) and runs TT*EE*CPL fma chains.
-template <int TT, int EE, int CPL>
+// It is memory latency: steps are loaded U at a time, one batch ahead of the
+// chains and the first ahead of the sums of squares (the feed-forward block
+// against a load round trip per step: 1 token 50.6 -> 47.9 us, 16 tokens 110.7
+// -> 103.5, 333 tokens 273 -> 252).
+template <int TT, int EE, int CPL, int U>
 __global__ __launch_bounds__(256) void k_router_logits(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ proj,
     const uint16_t* __restrict__ rscale, float* __restrict__ logits, int T, int H, int E,
@@ -38,25 +42,40 @@ __global__ __launch_bounds__(256) void k_router_logits(
   __shared__ float s_inv[TT];
   const int wave = threadIdx.x >> 6, lane = lane_id();
   const int t0 = blockIdx.x * TT, e0 = (blockIdx.y * 4 + wave) * EE;
+  constexpr int C = 64 * CPL;  // chains = PU*16 elements per step
+  const int iters = H / C;
+  using raw_t = std::conditional_t<CPL == 2, uint32_t, uint16_t>;
+  const uint16_t* xr[TT];
+  const uint16_t* wr[EE];
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) xr[tt] = x + (size_t)min(t0 + tt, T - 1) * H + lane * CPL;
+#pragma unroll
+  for (int ee = 0; ee < EE; ++ee) wr[ee] = proj + (size_t)min(e0 + ee, E - 1) * H + lane * CPL;
+  struct Batch { raw_t s[U], x[U][TT], w[U][EE]; };
+  auto load = [&](Batch& b, int i0) {  // (steps past the last repeat it, unused)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int off = min(i0 + u, iters - 1) * C;
+      b.s[u] = *reinterpret_cast<const raw_t*>(rscale + off + lane * CPL);
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) b.x[u][tt] = *reinterpret_cast<const raw_t*>(xr[tt] + off);
+#pragma unroll
+      for (int ee = 0; ee < EE; ++ee) b.w[u][ee] = *reinterpret_cast<const raw_t*>(wr[ee] + off);
+    }
+  };
+  Batch b0, b1;
+  if (iters > 0) load(b0, 0);
   for (int tt = wave; tt < TT; tt += 4) {
     const int t = min(t0 + tt, T - 1);
     const float ssq =
         wave_row_ssq(reinterpret_cast<const uint32_t*>(x + (size_t)t * H), H, pu_bf16);
     if (lane == 0) s_inv[tt] = sqrt_n / __builtin_sqrtf(ssq + n_eps);
   }
-  __syncthreads();
+  lds_barrier();
   float inv[TT];
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt) inv[tt] = s_inv[tt];
 
-  const uint16_t* xr[TT];
-  const uint16_t* wr[EE];
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt) xr[tt] = x + (size_t)min(t0 + tt, T - 1) * H;
-#pragma unroll
-  for (int ee = 0; ee < EE; ++ee) wr[ee] = proj + (size_t)min(e0 + ee, E - 1) * H;
-
-  constexpr int C = 64 * CPL;  // chains = PU*16 elements per step
   float acc[TT][EE][CPL];
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt)
@@ -65,79 +84,79 @@ __global__ __launch_bounds__(256) void k_router_logits(
 #pragma unroll
       for (int r = 0; r < CPL; ++r) acc[tt][ee][r] = 0.0f;
 
-  const int iters = H / C;
-  for (int i = 0; i < iters; ++i) {
-    const int off = i * C + lane * CPL;
-    float sv[CPL], xs[TT][CPL], wv[EE][CPL];
-    if constexpr (CPL == 2) {
-      const uint32_t s2 = *reinterpret_cast<const uint32_t*>(rscale + off);
-      sv[0] = __uint_as_float(s2 << 16);
-      sv[1] = __uint_as_float(s2 & 0xFFFF0000u);
+  auto widen = [](raw_t v, float (&f)[CPL]) {
+    f[0] = __uint_as_float((uint32_t)v << 16);
+    if constexpr (CPL == 2) f[1] = __uint_as_float((uint32_t)v & 0xFFFF0000u);
+  };
+  auto chains = [&](const Batch& b, int i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i0 + u >= iters) break;  // uniform
+      float sv[CPL], xs[TT][CPL];
+      widen(b.s[u], sv);
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
-        const uint32_t v = *reinterpret_cast<const uint32_t*>(xr[tt] + off);
-        xs[tt][0] = __uint_as_float(v << 16);
-        xs[tt][1] = __uint_as_float(v & 0xFFFF0000u);
+        widen(b.x[u][tt], xs[tt]);
+#pragma unroll
+        for (int r = 0; r < CPL; ++r) xs[tt][r] = xs[tt][r] * sv[r] * inv[tt];
       }
 #pragma unroll
       for (int ee = 0; ee < EE; ++ee) {
-        const uint32_t v = *reinterpret_cast<const uint32_t*>(wr[ee] + off);
-        wv[ee][0] = __uint_as_float(v << 16);
-        wv[ee][1] = __uint_as_float(v & 0xFFFF0000u);
+        float wv[CPL];
+        widen(b.w[u][ee], wv);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+          for (int r = 0; r < CPL; ++r) acc[tt][ee][r] = fmaf(xs[tt][r], wv[r], acc[tt][ee][r]);
       }
-    } else {
-      sv[0] = bf16_to_f32(rscale[off]);
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) xs[tt][0] = bf16_to_f32(xr[tt][off]);
-#pragma unroll
-      for (int ee = 0; ee < EE; ++ee) wv[ee][0] = bf16_to_f32(wr[ee][off]);
     }
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-      for (int r = 0; r < CPL; ++r) xs[tt][r] = xs[tt][r] * sv[r] * inv[tt];
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-      for (int ee = 0; ee < EE; ++ee)
-#pragma unroll
-        for (int r = 0; r < CPL; ++r) acc[tt][ee][r] = fmaf(xs[tt][r], wv[ee][r], acc[tt][ee][r]);
+  };
+  for (int i0 = 0; i0 < iters; i0 += 2 * U) {
+    if (i0 + U < iters) load(b1, i0 + U);
+    chains(b0, i0);
+    if (i0 + U >= iters) break;
+    if (i0 + 2 * U < iters) load(b0, i0 + 2 * U);
+    chains(b1, i0 + U);
   }
 
   // chain c = l*CPL + r is (p, j) = (c >> 4, c & 15).  tree_merge_accs
   // (simd_math/matrixops.mojo:265-283): acc[p] += acc[p + s] for s = 1, 2,
   // 4 -> partner lane + s*16/CPL; then the 16-lane halving reduce_add: lane
-  // + h/CPL for h >= CPL, in-lane r + 1 for h = 1 < CPL.  Lane 0, r = 0 ends
-  // with the logit; lane tt*EE + ee stores it.
-  constexpr int PU = 4 * CPL;
+  // + h/CPL for h >= CPL, in-lane r + 1 for h = 1 < CPL.  Partners 16 and 32
+  // lanes up are other rows: four logits share those two steps, exchanged so
+  // that logit 4 g + q ends in lane 0 of row q; lane g of that row keeps it.
+  static_assert(TT * EE <= 64 && TT * EE % 4 == 0, "one logit per lane, four at a time");
   float mine = 0.0f;
+  auto group = [&](auto gc) {
+    constexpr int g = decltype(gc)::value;
+    float t[CPL];
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-    for (int ee = 0; ee < EE; ++ee) {
-      float v[CPL];
-#pragma unroll
-      for (int r = 0; r < CPL; ++r) v[r] = acc[tt][ee][r];
-#pragma unroll
-      for (int q = 0; (1 << q) < PU; ++q)
-#pragma unroll
-        for (int r = 0; r < CPL; ++r) v[r] = v[r] + __shfl_down(v[r], (16 << q) / CPL, kWave);
+    for (int r = 0; r < CPL; ++r) {
+      float v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int h = 8 >> q;
-        if (h >= CPL) {
-#pragma unroll
-          for (int r = 0; r < CPL; ++r) v[r] = v[r] + __shfl_down(v[r], h / CPL, kWave);
-        } else if constexpr (CPL == 2) {
-          v[0] = v[0] + v[1];
-        }
+        v[q] = acc[(4 * g + q) / EE][(4 * g + q) % EE][r];
+        if constexpr (CPL == 2) v[q] = row_add_shl<8>(v[q]);
       }
-      const float total = __shfl(v[0], 0, kWave);
-      if (lane == tt * EE + ee) mine = total;
+      float lo, hi, x01, x23;
+      row_exchange<16>(v[0], v[1], lo, hi);
+      x01 = lo + hi;
+      row_exchange<16>(v[2], v[3], lo, hi);
+      x23 = lo + hi;
+      row_exchange<32>(x01, x23, lo, hi);
+      t[r] = lo + hi;
+      if constexpr (CPL == 1) t[r] = row_add_shl<8>(t[r]);
+      t[r] = row_add_shl<1>(row_add_shl<2>(row_add_shl<4>(t[r])));
     }
-  static_assert(TT * EE <= 64, "one logit per lane");
-  const int tt = lane / EE, ee = lane % EE;
-  if (lane < TT * EE && t0 + tt < T && e0 + ee < E) logits[(size_t)(t0 + tt) * E + e0 + ee] = mine;
+    float total = t[0];
+    if constexpr (CPL == 2) total = total + t[1];
+    if constexpr (g > 0)
+      total = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(total), 0x110 + g, 0xF, 0xF, true));
+    if ((lane & 15) == g) mine = total;
+  };
+  static_for<0, TT * EE / 4>(group);
+  const int idx = 4 * (lane & 15) + (lane >> 4), tt = idx / EE, ee = idx % EE;
+  if (idx < TT * EE && t0 + tt < T && e0 + ee < E) logits[(size_t)(t0 + tt) * E + e0 + ee] = mine;
 }
 
 // 64-bit key ordering candidates like insert_candidate: high word = the
@@ -499,17 +518,17 @@ static int pick_port_unroll(int width, int cols) {
   return 1;
 }
 
-template <int TT, int EE>
+template <int TT, int EE, int U>
 static hipError_t launch_logits_tile(const uint16_t* x, const uint16_t* proj,
                                      const uint16_t* rscale, float* logits, int T, int H, int E,
                                      float sqrt_n, float n_eps, hipStream_t st) {
   const dim3 grid((T + TT - 1) / TT, (E + 4 * EE - 1) / (4 * EE));
   const int pu_bf16 = pick_port_unroll(32, H);
   if (pick_port_unroll(16, H) == 8)
-    hipLaunchKernelGGL((k_router_logits<TT, EE, 2>), grid, dim3(256), 0, st, x, proj, rscale,
+    hipLaunchKernelGGL((k_router_logits<TT, EE, 2, U>), grid, dim3(256), 0, st, x, proj, rscale,
                        logits, T, H, E, pu_bf16, sqrt_n, n_eps);
   else
-    hipLaunchKernelGGL((k_router_logits<TT, EE, 1>), grid, dim3(256), 0, st, x, proj, rscale,
+    hipLaunchKernelGGL((k_router_logits<TT, EE, 1, U>), grid, dim3(256), 0, st, x, proj, rscale,
                        logits, T, H, E, pu_bf16, sqrt_n, n_eps);
   return hipGetLastError();
 }
@@ -517,8 +536,13 @@ static hipError_t launch_logits_tile(const uint16_t* x, const uint16_t* proj,
 hipError_t launch_router_logits(const uint16_t* x, const uint16_t* proj, const uint16_t* rscale,
                                 float* logits, int T, int H, int E, float sqrt_n, float n_eps,
                                 hipStream_t st) {
-  if (T >= 256) return launch_logits_tile<8, 8>(x, proj, rscale, logits, T, H, E, sqrt_n, n_eps, st);
-  return launch_logits_tile<2, 4>(x, proj, rscale, logits, T, H, E, sqrt_n, n_eps, st);
+  // larger tiles read fewer operand bytes per logit; smaller ones fill the chip
+  // (128 experts, the feed-forward block with 2 x 4 / 4 x 4 / 8 x 8 tiles: 16
+  // tokens 105.6 / 107.1 / 115.3 us, 150 tokens 191.3 / 189.5 / 199.4, 333
+  // tokens 259.9 / 252.3 / 259.6, 1400 tokens 455.9 / 431.8 / 430.8)
+  if (T >= 768) return launch_logits_tile<8, 8, 1>(x, proj, rscale, logits, T, H, E, sqrt_n, n_eps, st);
+  if (T >= 100) return launch_logits_tile<4, 4, 4>(x, proj, rscale, logits, T, H, E, sqrt_n, n_eps, st);
+  return launch_logits_tile<2, 4, 11>(x, proj, rscale, logits, T, H, E, sqrt_n, n_eps, st);
 }
 
 constexpr int kRouteScheduleFusedTokens = 8;

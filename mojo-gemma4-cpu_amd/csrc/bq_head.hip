@@ -188,8 +188,16 @@ __device__ inline void samp_merge(float& s, int& i, float os, int oi) {
   }
 }
 
-template <int MI, int CH>
+// NV: the logits of a strip that a lane finishes (softcap, Gumbel, log-sum-
+// exp: about 250 vector instructions each).  The MFMA leaves it rows 4 g + v
+// of one column; up to 8 rows half the lanes, up to 4 rows three quarters,
+// would finish rows that are not there, so the rows are first spread over the
+// lane groups (NV = 2: rows 4 (g & 1) + 2 (g >> 1) + v, NV = 1: row g).
+// The call with 262144 rows of vocabulary: 8 tokens 202 -> 189 us, 4 tokens
+// 193 -> 174.
+template <int MI, int CH, int NV>
 __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
+  static_assert(NV == 4 || MI == 1, "rows are spread from one MFMA tile");
   constexpr int RP = 16 * MI;  // padded rows
   const int wave = threadIdx.x >> 6, lane = lane_id();
   const int H = a.H, K64 = H >> 6, nb = H / a.block, fpb = a.block >> 6;
@@ -257,13 +265,17 @@ __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
   // (not __syncthreads: its fence would wait for the chunk loads in flight)
   lds_barrier();
 
-  // running partials per (mi, v) row slot: rows 16*mi + 4*(lane>>4) + v
-  float best[MI][4], lmx[MI][4], lsum[MI][4];
-  int bidx[MI][4];
+  auto row_of = [&](int mi, int v) {
+    const int g = lane >> 4;
+    return NV == 4 ? 16 * mi + 4 * g + v : NV == 2 ? 4 * (g & 1) + 2 * (g >> 1) + v : g;
+  };
+  // running partials per (mi, v) row slot
+  float best[MI][NV], lmx[MI][NV], lsum[MI][NV];
+  int bidx[MI][NV];
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
+    for (int v = 0; v < NV; ++v) {
       best[mi][v] = kNegInf;
       bidx[mi][v] = 0x7FFFFFFF;
       lmx[mi][v] = kNegInf;
@@ -310,13 +322,33 @@ __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
     // the strip's epilogue: y = bf16(softcap(raw)), score = y/T + gumbel
     const int col = (s0 + si * stride) * 16 + (lane & 15);  // this lane's vocabulary row
     const int64_t gidx = a.vbase + col;
+    float fin[MI][NV];
+    if constexpr (NV == 4) {
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) fin[mi][v] = raw[mi][v];
+    } else {
+      float x0, x1, unused;
+      row_exchange<32>(raw[0][0], raw[0][2], x0, unused);  // groups 2, 3: values 2 of 0, 1
+      row_exchange<32>(raw[0][1], raw[0][3], x1, unused);
+      if constexpr (NV == 2) {
+        fin[0][0] = x0;
+        fin[0][1] = x1;
+      } else {
+        row_exchange<16>(x0, x1, fin[0][0], unused);
+      }
+    }
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = 16 * mi + 4 * (lane >> 4) + v;
-        const float rv = raw[mi][v];
-        raw[mi][v] = 0.0f;
+      for (int v = 0; v < 4; ++v) raw[mi][v] = 0.0f;
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const int r = row_of(mi, v);
+        const float rv = fin[mi][v];
         if (r >= a.R) continue;
         const uint16_t yb = f32_to_bf16(tanh_f32(rv / a.cap) * a.cap);
         a.y[(size_t)r * a.V + col] = yb;
@@ -340,7 +372,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
+    for (int v = 0; v < NV; ++v) {
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) {
         const float os = __shfl_xor(best[mi][v], o, 16);
@@ -359,7 +391,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
         samp_merge(best[mi][v], bidx[mi][v], os, oi);
       }
       if ((lane & 15) == 0) {
-        const int r = 16 * mi + 4 * (lane >> 4) + v;
+        const int r = row_of(mi, v);
         s_red[wave][0][r] = best[mi][v];
         s_red[wave][1][r] = __int_as_float(bidx[mi][v]);
         s_red[wave][2][r] = lmx[mi][v];
@@ -367,7 +399,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void k_head_logits(HeadArgs a) {
       }
     }
   __syncthreads();
-  if (threadIdx.x < RP) {
+  if (threadIdx.x < 4 * NV * MI) {
     const int r = threadIdx.x;
     float bs = kNegInf, mx = kNegInf, sm = 0.0f;
     int bi = 0x7FFFFFFF;
@@ -911,14 +943,18 @@ hipError_t launch_flash_sample(const int8_t* x, const float* xsa, const int8_t* 
   // chunks of 4 fragments up to block 256 (104 VGPRs, two slots of 4 KiB
   // per wave), else 8 (a block never spans two chunks)
   const bool ch4 = block <= 256;
-  if (R <= 16 && ch4)
-    hipLaunchKernelGGL((k_head_logits<1, 4>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a);
-  else if (R <= 16)
-    hipLaunchKernelGGL((k_head_logits<1, 8>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a);
-  else if (ch4)
-    hipLaunchKernelGGL((k_head_logits<2, 4>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a);
-  else
-    hipLaunchKernelGGL((k_head_logits<2, 8>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a);
+#define BQ_HL(MI, NV)                                                                            \
+  do {                                                                                           \
+    if (ch4)                                                                                     \
+      hipLaunchKernelGGL((k_head_logits<MI, 4, NV>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a); \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_head_logits<MI, 8, NV>), dim3(grid), dim3(64 * kHeadWaves), lds, st, a); \
+  } while (0)
+  if (R <= 4) BQ_HL(1, 1);
+  else if (R <= 8) BQ_HL(1, 2);
+  else if (R <= 16) BQ_HL(1, 4);
+  else BQ_HL(2, 4);
+#undef BQ_HL
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
 

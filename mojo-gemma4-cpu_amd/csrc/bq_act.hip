@@ -389,9 +389,8 @@ __global__ __launch_bounds__(512) void k_norm_quant_pair(
 // Norm-quant with FWHT block 128, one wave per token (nq_v8_token): the
 // transform on 8 consecutive values per lane, so a 128-value block is one
 // row of 16 lanes and the FWHT's strides 1, 2, 4 run inside the lane and
-// strides 8, 16, 32, 64 across lanes 1, 2, 4, 8 apart (one DPP row move
-// each, two for lanes 4 apart) -- the reference's stages in its order, with
-// no cross-row swaps.
+// strides 8, 16, 32, 64 across lanes of the row (dpp_bfly8) -- the
+// reference's stages in its order, with no cross-row swaps.
 template <int NSEG>
 __global__ __launch_bounds__(256) void k_norm_quant_v8(
     const uint16_t* __restrict__ src, const uint16_t* __restrict__ gamma,
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(512) void k_norm_quant_v8_row(
 #pragma unroll
   for (int q = 0; q < NSEG; ++q)
     if (q < nseg) xp[q] = xr[64 * q];
-  const int e0 = 512 * wave + 8 * lane;
+  const int e0 = 512 * wave + 8 * dpp_run(lane);
   const int ec = min(e0, hidden - 8);  // runs past the row are read, never stored
   const v4i xv = *reinterpret_cast<const v4i*>(row + ec);
   const v4i gv = *reinterpret_cast<const v4i*>(gamma + ec);
@@ -510,16 +509,18 @@ hipError_t launch_norm_quant(const uint16_t* src, const uint16_t* gamma, int8_t*
     // many tokens: one wave each (4 per workgroup); few: a token over up to
     // 8 waves of SPW segments (a multiple of B/128 segments: whole blocks)
     // FWHT block 128: 8 values per lane for the transform (16-byte aligned
-    // gain, 8-byte aligned codes); a workgroup per token below 256 tokens
+    // gain, 8-byte aligned codes); a workgroup per token below 320 tokens (with
+    // a linear, hidden 2816, 256 tokens 16.9 us against 17.7 with a wave per
+    // token; hidden 4096, 333 tokens 22.2 / 22.0)
     const bool v8 = block == 128 && tune().nq_v8 && !(reinterpret_cast<uintptr_t>(gamma) & 15u) &&
                     !(reinterpret_cast<uintptr_t>(xq) & 7u);
-    if (v8 && seq_len < 256) {
+    if (v8 && seq_len < 320) {
       const dim3 g(seq_len), b(64 * ((hidden + 511) / 512));
 #define BQ_NQ8R(N) if (ns <= N) { hipLaunchKernelGGL((k_norm_quant_v8_row<N>), g, b, 0, st, src, gamma, xq, sa, hidden, sqrt_n, n_eps, sc); return hipGetLastError(); }
       BQ_NQ8R(8) BQ_NQ8R(16) BQ_NQ8R(22) BQ_NQ8R(24) BQ_NQ8R(32)
 #undef BQ_NQ8R
     }
-    if (v8 && seq_len >= 256) {
+    if (v8) {
       const dim3 g((seq_len + 3) / 4), b(256);
 #define BQ_NQ8(N) if (ns <= N) { hipLaunchKernelGGL((k_norm_quant_v8<N>), g, b, 0, st, src, gamma, xq, sa, seq_len, hidden, sqrt_n, n_eps, sc); return hipGetLastError(); }
       BQ_NQ8(8) BQ_NQ8(16) BQ_NQ8(22) BQ_NQ8(24) BQ_NQ8(32)

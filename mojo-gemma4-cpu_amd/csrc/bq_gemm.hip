@@ -568,7 +568,7 @@ __device__ __forceinline__ void norm_linear_skinny(const Args& args, const NormA
 #pragma unroll
   for (int q = 0; q < NSEG; ++q)  // first: the sum of squares needs it first
     if (q < nseg) xp[q] = xr[64 * q];
-  const int e0 = 512 * wave + 8 * lane;  // V8: this lane's run
+  const int e0 = 512 * wave + 8 * dpp_run(lane);  // V8: this lane's run
   if constexpr (V8) {
     const int ec = min(e0, K - 8);  // runs past the row are read, never used
     xv = *reinterpret_cast<const v4i*>(nq.src + ec);

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(512) void k_head_prep_v8(
 #pragma unroll
   for (int q = 0; q < NSEG; ++q)
     if (q < nseg) xp[q] = xr[64 * q];
-  const int e0 = 512 * wave + 8 * lane;
+  const int e0 = 512 * wave + 8 * dpp_run(lane);
   const int ec = min(e0, hidden - 8);  // runs past the row are read, never stored
   const v4i xv = *reinterpret_cast<const v4i*>(row + ec);
   const v4i gv = *reinterpret_cast<const v4i*>(gamma + ec);

@@ -132,3 +132,9 @@ def test_embed_lookup(gpu, O, H, B):
                                                         ws[48 * rank:48 * rank + 48], B,
                                                         scale=scale, shard_rows=48, rank=rank))
         assert (g[:6] == 0).all()
+
+
+@pytest.mark.parametrize("R", [4, 5, 8, 9, 16])
+def test_flash_sample_row_spread(gpu, O, R):
+    # one, two and four rows per lane in the logits kernel's epilogue
+    test_flash_sample(gpu, O, R, 2048, 512, False)

@@ -805,3 +805,16 @@ def test_moe_model_shape_decode(gpu, O, moe_model):
     np.testing.assert_array_equal(host(accum), racc)
     np.testing.assert_array_equal(host(out), rout)
     tol_check(host(accum), racc)
+
+
+@pytest.mark.parametrize("T", [1, 319, 320])  # fused-size row, a workgroup per token, a wave per token
+def test_norm_quant_tiny_rows(gpu, O, T):
+    # gains so small that 127 / amax overflows, beside ordinary rows
+    x = O.synth_normal_bf16(9, 1.0, (T, 2816))
+    x[T // 2] = 0
+    for g in (0x0080, 0x0200, ONE):
+        gamma = np.full(2816, g, np.uint16)
+        q, sa = gpu.norm_quant(dev(x), dev(gamma), 128)
+        rq, rsa = O.norm_quant(x, gamma, 128)
+        np.testing.assert_array_equal(host(sa).view(np.uint32), rsa.view(np.uint32))
+        np.testing.assert_array_equal(host(q), rq)

@@ -98,3 +98,11 @@ def test_router_to_schedule(gpu, O):
     np.testing.assert_array_equal(r[:, 0], rroutes["token"])
     np.testing.assert_array_equal(r[:, 1].view(np.float32).view(np.uint32),
                                   rroutes["weight"].view(np.uint32))
+
+
+@pytest.mark.parametrize("T,H,E", [(99, 2816, 70), (100, 2816, 70), (101, 320, 16), (767, 1408, 33),
+                                   (768, 1408, 33), (769, 2944, 130)])
+def test_router_logits_tiles(gpu, O, T, H, E):
+    # around the tile sizes' boundaries: ragged last tiles, one and two chains
+    # per lane, step counts that leave part of a batch
+    test_router_logits(gpu, O, T, H, E)

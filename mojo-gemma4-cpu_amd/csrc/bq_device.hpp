@@ -769,12 +769,11 @@ __device__ inline void codes8_bounded(const float (&v)[8], float inv, uint32_t (
 }
 
 // ---------------------------------------------------------------------------
-// Norm-quant transform with FWHT block 128 on 8 consecutive values per lane
-// (lane L of a 512-value round holds run l = dpp_run(L), values 8l .. 8l+7, so
-// a 128-value block is one row of 16 lanes): x * inv_rms * gain, the FWHT's
-// strides 1, 2, 4 inside the lane and strides 8, 16, 32, 64 across lanes
-// (dpp_bfly8: one instruction per value and stage), times fwht_scale -- the
-// reference's stages in its order.  Each cross-lane
+// FWHT of 128-value blocks on 8 consecutive values per lane (lane L of a
+// 512-value round holds run l = dpp_run(L), values 8l .. 8l+7, so a block is
+// one row of 16 lanes), times fwht_scale: strides 1, 2, 4 inside the lane,
+// strides 8, 16, 32, 64 across lanes (dpp_bfly8: one instruction per value and
+// stage) -- the reference's stages in its order.  Each cross-lane
 // stage computes own + s * partner, s = -1 on the upper lane of a pair, so
 // the upper lane holds b - a = -(a - b); before every such stage both lanes
 // of a pair carry the same sign (the parity of the lane bits already
@@ -782,17 +781,11 @@ __device__ inline void codes8_bounded(const float (&v)[8], float inv, uint32_t (
 // (negation commutes with round-to-nearest), and the final sign,
 // (-1)^parity(l & 15), is folded into the scale multiply.  Returns the
 // lane's max |v|.
-__device__ inline float nq_v8_transform(v4i xv, v4i gv, float inv_rms, float fwht_scale,
-                                        float (&v)[8]) {
+__device__ inline float fwht128_v8(float fwht_scale, float (&v)[8]) {
   const int run = dpp_run(lane_id());
   const float s1 = (run & 1) ? -1.0f : 1.0f, s2 = (run & 2) ? -1.0f : 1.0f;
   const float s4 = (run & 4) ? -1.0f : 1.0f, s8 = (run & 8) ? -1.0f : 1.0f;
   const float sc_lane = (__builtin_popcount(run & 15) & 1) ? -fwht_scale : fwht_scale;
-  float xf[8], gf[8];
-  bf16x8_to_f32(xv, xf);
-  bf16x8_to_f32(gv, gf);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = xf[j] * inv_rms * gf[j];
 #pragma unroll
   for (int st = 1; st < 8; st <<= 1)
 #pragma unroll
@@ -813,6 +806,17 @@ __device__ inline float nq_v8_transform(v4i xv, v4i gv, float inv_rms, float fwh
     m = fmaxf(m, fabsf(v[j]));
   }
   return m;
+}
+
+// Norm-quant transform with FWHT block 128: x * inv_rms * gain, then the above.
+__device__ inline float nq_v8_transform(v4i xv, v4i gv, float inv_rms, float fwht_scale,
+                                        float (&v)[8]) {
+  float xf[8], gf[8];
+  bf16x8_to_f32(xv, xf);
+  bf16x8_to_f32(gv, gf);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = xf[j] * inv_rms * gf[j];
+  return fwht128_v8(fwht_scale, v);
 }
 
 // the 8 int8 codes of v, little-endian in two words

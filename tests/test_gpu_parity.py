@@ -818,3 +818,20 @@ def test_norm_quant_tiny_rows(gpu, O, T):
         rq, rsa = O.norm_quant(x, gamma, 128)
         np.testing.assert_array_equal(host(sa).view(np.uint32), rsa.view(np.uint32))
         np.testing.assert_array_equal(host(q), rq)
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 128), (3, 640), (9, 1024), (4, 2816), (7, 5632), (2, 6144),
+                                       (2, 6272)])
+@pytest.mark.parametrize("gain", [False, True])
+def test_quantize_weight_rows(gpu, O, rows, cols, gain):
+    # block 128, per-row: a wave per row up to 6144 values; part of a round, a
+    # row of zeros and one so small that 127 / amax overflows
+    w = O.synth_normal_bf16(cols, 0.02, (rows, cols))
+    w[1] = 0
+    w[rows - 1] = O.f32_to_bf16(O.bf16_to_f32(w[rows - 1]) * np.float32(1e-37))
+    f = O.bf16_to_f32(w)
+    g = np.random.default_rng(cols).uniform(0.5, 1.5, cols).astype(np.float32) if gain else None
+    q, s = gpu.quantize_weight(dev(w), 128, gamma=dev(g) if gain else None)
+    rq, rs = O.rotate_and_quant(f * g if gain else f, 128)
+    np.testing.assert_array_equal(host(s).view(np.uint32), rs.view(np.uint32))
+    np.testing.assert_array_equal(host(q), rq)

@@ -10,10 +10,11 @@
 //   per-block(gemm.mojo:194-215):  facc = fma(f32(acc_b), sa[m,b]*(1/127), facc)
 //                                  for b ascending;  y = facc * ws[n]
 //
-// k_linear_skinny (M <= 16, decode): one workgroup per 16-row n-tile, waves
+// k_linear_skinny (decode, and up to a few dozen rows): one workgroup per
+//   16-row n-tile and 16 rows, waves
 //   split K; each step streams one 1 KiB weight fragment per wave (HBM-bound,
 //   no LDS staging of weights).  Partial int32 tiles are reduced exactly in LDS.
-// M > 16 (prefill) runs the LDS-tiled kernel of bq_tiled.hip.
+// More rows (prefill) run the LDS-tiled kernel of bq_tiled.hip.
 #include "bq_device.hpp"
 #include "bq_kernels.hpp"
 
@@ -67,14 +68,16 @@ __device__ inline LinSeg seg_of(const Seg1Args& a, int& nt) {
 }
 
 // ---------------------------------------------------------------------------
-// skinny: M <= 16
+// skinny: 16 rows per workgroup
 // ---------------------------------------------------------------------------
 template <int WAVES, bool PER_BLOCK, int U, class Args>
 __device__ __forceinline__ void linear_skinny(const Args& args) {
   extern __shared__ int lds[];  // per-row: WAVES*256 ints; per-block: nb*256 ints
   int nt;
   const LinSeg seg = seg_of(args, nt);
-  const int K = args.K, K64 = K >> 6, M = args.M;
+  // rows 16 blockIdx.y .. of the call
+  const int m0 = 16 * blockIdx.y;
+  const int K = args.K, K64 = K >> 6, M = min(args.M - m0, 16);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int fpb = args.block >> 6;  // fragments per K block (power of two)
   const int nb = K / args.block;
@@ -110,12 +113,12 @@ __device__ __forceinline__ void linear_skinny(const Args& args) {
   // unmasked loads (clamped index): a masked load would make the compiler
   // wait for the whole weight stream at the branch join
   const float ews = seg.ws[en];
-  const float ead = PER_BLOCK ? 0.0f : args.sa[min(ei, M - 1)] * kInv127;
+  const float ead = PER_BLOCK ? 0.0f : args.sa[m0 + min(ei, M - 1)] * kInv127;
   // rows >= M load row 0 instead: accumulator row i depends only on A row i
   // and rows >= M are never stored, so the loads need no mask (a branch
   // around them would force the compiler to wait for every outstanding load)
   const bool arow = (lane & 15) < M;
-  const int8_t* ab = args.act + (size_t)(arow ? (lane & 15) : 0) * K + (lane >> 4) * 16;
+  const int8_t* ab = args.act + (size_t)(m0 + (arow ? (lane & 15) : 0)) * K + (lane >> 4) * 16;
   const v4i zero = {0, 0, 0, 0};
   v4i c = zero;
 
@@ -198,7 +201,7 @@ __device__ __forceinline__ void linear_skinny(const Args& args) {
   // epilogue: thread t <-> accumulator element (v = t/64, L = t%64):
   // row 4*(L/16)+v, column L%16 of the 16x16 tile.
   if (!eact) return;
-  const int i = ei, n = en;
+  const int i = m0 + ei, n = en;
   float y;
   if (PER_BLOCK) {
     float facc = 0.0f;
@@ -454,9 +457,21 @@ static void pick_linear_tile(const LinArgs& a, int per_block, int& bm, int& bn) 
 
 hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
   if (a.M <= 0) return hipSuccess;
-  if (a.M <= 16) {
-    int tiles = 0;
-    for (int q = 0; q < a.nseg; ++q) tiles += a.seg[q].n / 16;
+  // Past 16 rows the tiled kernels take over once they have workgroups enough:
+  // a few dozen rows over few columns leave most CUs idle there, where 16 x 16
+  // tiles with K split over 16 waves fill the chip, the weights read again from
+  // L2 for each 16 rows.  Per-row up to three such tiles per CU (with its
+  // norm-quant, 32 x 4096 at K 4096 25.9 -> 20.4 us, 64 x 1024 19.4 -> 14.0, but
+  // 48 x 8192 at K 2816 6 us longer), per-block up to six (32 x 2816 at K 8192
+  // 31 -> 12 us, 128 rows 1.3 us shorter).  (A switch of the tiled kernels
+  // keeps them.)
+  int tiles = 0;
+  for (int q = 0; q < a.nseg; ++q) tiles += a.seg[q].n / 16;
+  const int mtiles = (a.M + 15) / 16;
+  const bool skinny = a.M <= 16 || (mtiles <= 16 && tiles * mtiles <= (per_block ? 6 : 3) * tune().cus &&
+                                    a.K / a.block <= 64 && !tune().tile_bm && !tune().tile_bn &&
+                                    !tune().ring && !tune().tile_ksp);
+  if (skinny) {
     // M = 1 per-row up to K = 4096: k_gemv_m1 (BQ_GEMV_WAVES sends it to the
     // general kernel below)
     if (a.M == 1 && !per_block && !tune().gemv_waves && a.K <= 4096) {
@@ -480,7 +495,7 @@ hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
     // ceil(tiles / CUs) n-tiles per workgroup (at most 4, or BQ_SKINNY2 when
     // that is 2 or 3) while there are >= 2 per CU: one workgroup per CU, each
     // activation read shared by its tiles
-    if (!per_block && a.M >= 2 && !tune().gemv_waves && a.K <= 4096 && tune().skinny2 &&
+    if (!per_block && a.M >= 2 && a.M <= 16 && !tune().gemv_waves && a.K <= 4096 && tune().skinny2 &&
         tiles >= 2 * tune().cus) {
       const int cap = tune().skinny2 >= 2 ? min(tune().skinny2, 4) : 4;
       const int nt = min(cap, (tiles + tune().cus - 1) / tune().cus);
@@ -496,7 +511,7 @@ hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
     // layer 147.4 -> 145.8 us.
     const int waves = tune().gemv_waves ? tune().gemv_waves : 16;
     const int nb = a.K / a.block;
-    dim3 g(tiles);
+    dim3 g(tiles, mtiles);
     const Seg1Args s1 = seg1_args(a);
     const bool one = a.nseg == 1;
 #define BQ_GO(W, PB, U_)                                                                        \

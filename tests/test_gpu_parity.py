@@ -835,3 +835,26 @@ def test_quantize_weight_rows(gpu, O, rows, cols, gain):
     rq, rs = O.rotate_and_quant(f * g if gain else f, 128)
     np.testing.assert_array_equal(host(s).view(np.uint32), rs.view(np.uint32))
     np.testing.assert_array_equal(host(q), rq)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 127])
+@pytest.mark.parametrize("K,B", [(704, None), (4096, None), (1024, 256), (2112, 64), (8192, 512)])
+def test_linear_row_tiles(gpu, O, M, K, B):
+    # more than 16 rows in 16-row workgroups: a last tile of one row, of all,
+    # of all but one; one-shot and looping K slices
+    N = 96
+    q, s = O.rotate_and_quant(O.bf16_to_f32(O.synth_normal_bf16(3, 0.02, (N, K))), B or 64)
+    W = gpu.ButterquantWeight(gpu.retile(dev(q.reshape(-1)), N, K), dev(s), N, K)
+    x = O.synth_normal_bf16(4, 1.0, (M, K))
+    if B is None:
+        xq, sa = O.norm_quant(x, np.full(K, ONE, np.uint16), 64)
+        ob, of = gpu.linear(dev(xq), dev(sa), W, want_f32=True)
+        p, cs = O.pack_and_colsum(q)
+        rb, rf = O.linear(xq, sa, p, s, cs, N)
+    else:
+        xq, sa = O.block_quant(x, B, B == 64)
+        ob, of = gpu.block_linear(dev(xq), dev(sa), W, B, want_f32=True)
+        p, cs = O.pack_and_colsum(q, B, False)
+        rb, rf = O.block_linear(xq, sa, p, s, cs, N, B)
+    np.testing.assert_array_equal(host(of), rf)
+    np.testing.assert_array_equal(host(ob), rb)

@@ -675,12 +675,15 @@ __global__ __launch_bounds__(256, 2) void k_flash_attn(AttnArgs a) {
 // 400 vector instructions per wave.  The block of 2048 tokens from position 0
 // (sliding, head 256): 598 -> 412 us, attention alone 403 -> 222 us against a
 // wave per 8 tokens on v_fma; 700 + 411 tokens (full, head 512): 699 -> 396 us.
-template <int HD, int G>
-__global__ __launch_bounds__(256, HD >= 512 ? 2 : 3) void k_flash_attn_rows(AttnArgs a, int nblk) {
+// LONE: the instance of split plans whose blocks without a sliding window run
+// a wave per token; four waves per SIMD for those (200 tokens at position 500,
+// the block 140 -> 128 us), where the groups' own code wants the registers of
+// three (2048 tokens 330 us, with four 340).
+template <int HD, int G, bool LONE>
+__global__ __launch_bounds__(256, LONE ? 4 : HD >= 512 ? 2 : 3) void k_flash_attn_rows(AttnArgs a, int nblk) {
   constexpr int C = HD / 64;    // 64-byte K chunks per row; column tiles per wave
   constexpr int TPW = 16 / G;   // tokens per group
   constexpr int NL = G >= 4 ? 1 : 4 / G;  // tokens among a lane's four rows
-  constexpr int NH = attn_rows_parts(G);  // workgroups per group
   // a step's weights [position][row]; corrections, weight sums (row 4: a spare)
   // and maxima [tile][row]
   __shared__ __attribute__((aligned(16))) float s_w[64 * 16];
@@ -705,7 +708,11 @@ __global__ __launch_bounds__(256, HD >= 512 ? 2 : 3) void k_flash_attn_rows(Attn
   // between it would leave some shader engines idle)
   const int part = item / (nblk * 16);
   item -= part * nblk * 16;
-  const int cls = item % 16, t0 = (nblk - 1 - item / 16) * 16 * TPW;
+  // (every other block's groups in reverse: a CU takes every 32nd workgroup of
+  // its XCD, which would be the longest ranges of each block for some CUs and
+  // the shortest for others)
+  const int cls = (item / 16 + part) & 1 ? 15 - item % 16 : item % 16;
+  const int t0 = (nblk - 1 - item / 16) * 16 * TPW;
   const int run0 = run_of(a.runs, a.num_runs, t0);
   auto run_from = [&](int tok) {  // run_of(tok), tok >= t0
     int r = run0;
@@ -728,12 +735,12 @@ __global__ __launch_bounds__(256, HD >= 512 ? 2 : 3) void k_flash_attn_rows(Attn
     }
     if (__ballot(slides)) { tok0 = t0 + cls; step = 16; }
   }
-  if constexpr (NH > 1) {
+  if constexpr (LONE) {
     // Where nothing slides, two neighbours' splits start together only if
     // ceil(L / S) is the same for both: with fewer splits than tokens a group
     // would be several small sets, and a wave per token is faster (200 tokens
     // from position 0, two splits: the block 83 against 74 us)
-    if (step == 1 && attn_rows_lone(G, a.s_max)) {
+    if (step == 1) {
       const int tok = tok0 + 4 * part + wave;
       if (tok < a.T) flash_attn_wave<HD, G>(a, tok, kvh, s, s_w + wave * 16 * G);
       return;
@@ -1113,14 +1120,20 @@ static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
   // tokens share nothing: a wave each.
   const int tpw = 16 / gqa, nblk = (a.T + 16 * tpw - 1) / (16 * tpw);
   if (a.s_max == 1 || a.T >= 2 * tpw * a.num_runs) {
-    const int nh = attn_rows_lone(gqa, a.s_max) ? attn_rows_parts(gqa) : 1;
-    const dim3 g(nblk * 16 * nh * a.num_kv * a.s_max);
+    const bool lone = attn_rows_lone(gqa, a.s_max);
+    const dim3 g(nblk * 16 * (lone ? attn_rows_parts(gqa) : 1) * a.num_kv * a.s_max);
     switch (gqa) {
-      case 1: hipLaunchKernelGGL((k_flash_attn_rows<HD, 1>), g, b, 0, st, a, nblk); break;
-      case 2: hipLaunchKernelGGL((k_flash_attn_rows<HD, 2>), g, b, 0, st, a, nblk); break;
-      case 4: hipLaunchKernelGGL((k_flash_attn_rows<HD, 4>), g, b, 0, st, a, nblk); break;
-      case 8: hipLaunchKernelGGL((k_flash_attn_rows<HD, 8>), g, b, 0, st, a, nblk); break;
-      case 16: hipLaunchKernelGGL((k_flash_attn_rows<HD, 16>), g, b, 0, st, a, nblk); break;
+      case 1:
+        if (lone) hipLaunchKernelGGL((k_flash_attn_rows<HD, 1, true>), g, b, 0, st, a, nblk);
+        else hipLaunchKernelGGL((k_flash_attn_rows<HD, 1, false>), g, b, 0, st, a, nblk);
+        break;
+      case 2:
+        if (lone) hipLaunchKernelGGL((k_flash_attn_rows<HD, 2, true>), g, b, 0, st, a, nblk);
+        else hipLaunchKernelGGL((k_flash_attn_rows<HD, 2, false>), g, b, 0, st, a, nblk);
+        break;
+      case 4: hipLaunchKernelGGL((k_flash_attn_rows<HD, 4, false>), g, b, 0, st, a, nblk); break;
+      case 8: hipLaunchKernelGGL((k_flash_attn_rows<HD, 8, false>), g, b, 0, st, a, nblk); break;
+      case 16: hipLaunchKernelGGL((k_flash_attn_rows<HD, 16, false>), g, b, 0, st, a, nblk); break;
       default: return hipErrorInvalidValue;
     }
   } else {

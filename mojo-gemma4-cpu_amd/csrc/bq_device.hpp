@@ -296,7 +296,8 @@ __device__ inline float row_shl(float v) {
 }
 
 // v_max_f32 as it is: the larger, or the one that is a number (fmaxf would
-// first pass each operand through a canonicalizing v_max)
+// first pass each operand through a canonicalizing v_max).  For results that
+// plain vector instructions read: nothing waits for a cross-lane read of them.
 __device__ inline float max_num(float a, float b) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
@@ -307,14 +308,14 @@ __device__ inline float max_num(float a, float b) {
 // once: DPP row rotations by 8, 4, 2, 1 (max takes any order; a NaN loses to a
 // number).  In asm: fmaxf would first pass each moved value through a
 // canonicalizing v_max.  Four values in turn keep two instructions between a
-// write and the DPP read of it.
+// write and the DPP read of it; the last wait states as in dpp_bfly8.
 __device__ inline void row_max16_x4(float (&v)[4]) {
 #define BQ_ROR(n)                                                  \
   "v_max_f32_dpp %0, %0, %0 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
   "v_max_f32_dpp %1, %1, %1 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
   "v_max_f32_dpp %2, %2, %2 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t" \
   "v_max_f32_dpp %3, %3, %3 row_ror:" #n " row_mask:0xf bank_mask:0xf\n\t"
-  asm("s_nop 1\n\t" BQ_ROR(8) BQ_ROR(4) BQ_ROR(2) BQ_ROR(1) "s_nop 0"
+  asm("s_nop 1\n\t" BQ_ROR(8) BQ_ROR(4) BQ_ROR(2) BQ_ROR(1) "s_nop 1"
       : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
 #undef BQ_ROR
 }
@@ -697,7 +698,8 @@ __device__ inline float nq_pair_transform(const uint32_t (&x)[SPW], const uint32
 // (lane ^ 7), so index bit 2 is laid out as that: lane L holds run
 // dpp_run(L) = L ^ 3 where bit 2 of L is set, and s = -1 where dpp_run's bit
 // is set.  Eight values in turn keep every write eight instructions from the
-// DPP read of it.
+// DPP read of it; the wait states at the end are those of a DPP or lane-swap
+// read that follows (the compiler does not count them from writes in asm).
 __device__ inline int dpp_run(int lane) { return lane & 4 ? lane ^ 3 : lane; }
 
 template <int ST>
@@ -711,7 +713,8 @@ __device__ inline void dpp_bfly8(float (&v)[8], float s) {
       "v_fmac_f32_dpp %4, %4, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
       "v_fmac_f32_dpp %5, %5, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
       "v_fmac_f32_dpp %6, %6, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
-      "v_fmac_f32_dpp %7, %7, %8 " ctrl " row_mask:0xf bank_mask:0xf"                           \
+      "v_fmac_f32_dpp %7, %7, %8 " ctrl " row_mask:0xf bank_mask:0xf\n\t"                       \
+      "s_nop 1"                                                                                 \
       : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]),     \
         "+v"(v[7])                                                                              \
       : "v"(s))

@@ -30,8 +30,6 @@
 // split order with the reference's merge (corrections masked by l > 0, a
 // 16-lane tree per batch of 16 splits, the first contributing split
 // multiplied, the rest fma-accumulated).
-#include <type_traits>
-
 #include "bq_kernels.hpp"
 #include "bq_device.hpp"
 
@@ -471,12 +469,12 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
   };
   // One tile's operands: lane (p + 16 g) holds K row p's bytes [c*64 + g*16,
   // +16) for every chunk c, its ks and vs; every lane holds its C bytes of
-  // each V row.  Idle positions repeat the tile's first row.  Up to two heads,
-  // each register is requested again, for the next tile, as soon as this tile
-  // has used it (AHEAD): a wave waits for memory once, not once per tile.  With
-  // more heads the registers this takes cost more than the wait (16 sequences
-  // of 4096 positions, head 512: the block 91 -> 111 us).
-  constexpr bool AHEAD = G <= 2;
+  // each V row.  Idle positions repeat the tile's first row.  (Requesting the
+  // next tile's registers as this tile frees them measured slower: the waves of
+  // a SIMD already cover each other's loads.  Sliding, head 256, two heads per
+  // kv head, caches not in L2: 16 x 1000 positions 24.5 us against 23.4, 32
+  // 36.0 / 34.1, one sequence 12.3 / 12.0; head 512, eight heads, the registers
+  // it takes: a decode block 91 -> 111.)
   v4i kb[C];
   uint32_t vraw[16][(C + 3) / 4];
   float ks, vs;
@@ -503,26 +501,28 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
     }
   };
 
+  // The batch after is requested ahead, behind a tile's loads: a branch in
+  // front of them holds them back (128 sequences of 1500 positions, sliding:
+  // 124 us against 108).  Head 512 with a query head of its own per kv head is
+  // bound by HBM and takes its batches when due: a fourth wave per SIMD fits
+  // its registers then (8 sequences of 3000 positions, 16 heads: 77 us, 81 ahead).
+  constexpr bool NEXT = HD / G < 512;
   int off = 0, slots = 0, slots_n = 0;  // the next tile: its batch, and the batch after
   if (start < end) {
     slots = slot_batch(start);
-    slots_n = slot_batch(start + 64);
-    if constexpr (AHEAD) {
-      load_k(slots, 0, end - start);
-#pragma unroll
-      for (int p = 0; p < 16; ++p) load_v(p, slots, 0, end - start);
-    }
+    if constexpr (NEXT) slots_n = slot_batch(start + 64);
   }
   for (int p0 = start; p0 < end; p0 += 16) {
     const int tl = end - p0 < 16 ? end - p0 : 16;
-    const int tl_n = end - p0 - 16;  // of the next tile; <= 0: there is none
-    if constexpr (!AHEAD) {
-      load_k(slots, off, tl);
-#pragma unroll
-      for (int p = 0; p < 16; ++p) load_v(p, slots, off, tl);
+    if (!NEXT && off == 64) {
+      off = 0;
+      slots = slot_batch(p0);
     }
+    load_k(slots, off, tl);
+#pragma unroll
+    for (int p = 0; p < 16; ++p) load_v(p, slots, off, tl);
     off += 16;
-    if (off == 64) {
+    if (NEXT && off == 64) {
       off = 0;
       slots = slots_n;
       slots_n = slot_batch(p0 + 80);
@@ -530,8 +530,6 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
     v4i d = zero4;
 #pragma unroll
     for (int c = 0; c < C; ++c) d = mfma16x16x64(qa[c], kb[c], d);
-    const float ks_t = ks, vs_t = vs;
-    if (AHEAD && tl_n > 0) load_k(slots, off, tl_n);
     const int dv[4] = {d.x, d.y, d.z, d.w};
     // per head of this lane's group (heads 4 g + i, only i < G exist)
     constexpr int NI = G < 4 ? G : 4;
@@ -540,14 +538,14 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
     for (int i = 0; i < NI; ++i) {
       float sco = -1e30f;
       if (4 * grp + i < G && p16 < tl)
-        sco = (((float)(dv[i] + qsum128[i]) - qb[i]) * fq[i]) * ks_t * inv127sq;
+        sco = (((float)(dv[i] + qsum128[i]) - qb[i]) * fq[i]) * ks * inv127sq;
       const float tmax = group_max(sco, 16);
       const float m_new = tmax > m[i] ? tmax : m[i];
       corr[i] = fast_exp_softmax_biased(max87(m[i] - m_new));
       const float w = fast_exp_softmax_biased(max87(sco - m_new));
       l[i] = l[i] * corr[i] + tree16(w);
       m[i] = m_new;
-      sc[i] = p16 < tl ? w * vs_t * inv127 : 0.0f;
+      sc[i] = p16 < tl ? w * vs * inv127 : 0.0f;
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
@@ -571,33 +569,28 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
       for (int i = 0; i < NI; ++i)
         if (grp == 0) wsh[p16 * G + i] = sc[i];
     }
-    auto update = [&](auto reload) {
 #pragma unroll
-      for (int p = 0; p < 16; ++p) {
-        float vf[C];
+    for (int p = 0; p < 16; ++p) {
+      float vf[C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) vf[c] = (float)(int8_t)(vraw[p][c / 4] >> (8 * (c % 4)));
-        if constexpr (decltype(reload)::value) load_v(p, slots, off, tl_n);
-        if constexpr (G >= 4) {
-          float w[HB];
+      for (int c = 0; c < C; ++c) vf[c] = (float)(int8_t)(vraw[p][c / 4] >> (8 * (c % 4)));
+      if constexpr (G >= 4) {
+        float w[HB];
 #pragma unroll
-          for (int b = 0; b < HB; ++b) w[b] = wsh[p * G + (lane & 3) * HB + b];
+        for (int b = 0; b < HB; ++b) w[b] = wsh[p * G + (lane & 3) * HB + b];
 #pragma unroll
-          for (int b = 0; b < HB; ++b)
+        for (int b = 0; b < HB; ++b)
 #pragma unroll
-            for (int c = 0; c < C; ++c) acc[b][c] = mfma4x64x1f(w[b], vf[c], acc[b][c]);
-        } else {
+          for (int c = 0; c < C; ++c) acc[b][c] = mfma4x64x1f(w[b], vf[c], acc[b][c]);
+      } else {
 #pragma unroll
-          for (int h = 0; h < G; ++h) {
-            const float w = wsh[p * G + h];
+        for (int h = 0; h < G; ++h) {
+          const float w = wsh[p * G + h];
 #pragma unroll
-            for (int c = 0; c < C; ++c) acc[0][c][h] = fmaf(vf[c], w, acc[0][c][h]);
-          }
+          for (int c = 0; c < C; ++c) acc[0][c][h] = fmaf(vf[c], w, acc[0][c][h]);
         }
       }
-    };
-    if (AHEAD && tl_n > 0) update(std::true_type{});
-    else update(std::false_type{});
+    }
   }
 
   // finished here: a sliding token with one split (acc * (1/l)), and every
@@ -639,8 +632,11 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
   }
 }
 
+// Two waves per SIMD keep the accumulators out of the AGPRs (head 512, eight
+// heads: 16 sequences of 4096 positions 61.6 -> 53.4 us); head 512 with sixteen
+// does not fit the registers of two (36 spilled: 38.9 us against 33.5 with one).
 template <int HD, int G>
-__global__ __launch_bounds__(256, 2) void k_flash_attn(AttnArgs a) {
+__global__ __launch_bounds__(256, HD * G >= 8192 ? 1 : 2) void k_flash_attn(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) float s_w[4][16 * G];
   const int wave = threadIdx.x >> 6;
   const int per_tok = a.num_kv * a.s_max;

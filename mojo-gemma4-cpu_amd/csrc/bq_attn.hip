@@ -1145,16 +1145,18 @@ static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
     }
   }
   if (a.s_max == 1) return hipGetLastError();  // every token finished in the wave
-  // up to 8 splits (many tokens): two columns per lane and as many rows in
-  // flight as the plan can have; more splits (few tokens): one column, 32 rows
-  // (64 splits, 16 tokens, head 512: 9.7 us; with the rows staged in LDS for one
-  // wave's chain 16.9)
+  // up to 16 splits: two columns per lane and as many rows in flight as the
+  // plan can have (16 sequences of 1024 positions, sliding, 16 splits: the two
+  // attention kernels 24.4 us, with 32 rows 25.0); more splits (few tokens):
+  // one column, 32 rows (64 splits, 16 tokens, head 512, partials not in L2:
+  // 9.8 us; with the rows staged in LDS for one wave's chain 16.6)
   constexpr int CL = HD >= 128 ? 2 : 1;
   const int waves = a.T * a.num_q * (HD / 64);
   const dim3 g2((waves / CL + 3) / 4), g1((waves + 3) / 4);
   if (a.s_max <= 2) hipLaunchKernelGGL((k_attn_merge<HD, 2, CL>), g2, b, 0, st, a);
   else if (a.s_max <= 4) hipLaunchKernelGGL((k_attn_merge<HD, 4, CL>), g2, b, 0, st, a);
   else if (a.s_max <= 8) hipLaunchKernelGGL((k_attn_merge<HD, 8, CL>), g2, b, 0, st, a);
+  else if (a.s_max <= 16) hipLaunchKernelGGL((k_attn_merge<HD, 16, CL>), g2, b, 0, st, a);
   else hipLaunchKernelGGL((k_attn_merge<HD, 32, 1>), g1, b, 0, st, a);
   return hipGetLastError();
 }

@@ -241,3 +241,13 @@ def test_attn_prep_many_tokens(gpu, O, hd, rope_half, nq, nkv, degree, rank, nto
         np.testing.assert_array_equal(host(x).view(np.uint8), y.view(np.uint8))
     for n in ("kc", "ks", "vc", "vs"):
         np.testing.assert_array_equal(host(g[n]).view(np.uint8), p[n].view(np.uint8))
+
+
+@pytest.mark.parametrize("hd", [64, 128, 512])
+@pytest.mark.parametrize("s_max", [2, 3, 4, 5, 8, 9, 16, 17])
+def test_attention_merge_instances(gpu, O, hd, s_max):
+    # the fewest and the most splits of each merge instance, and tokens with
+    # fewer splits than the plan
+    c = make_case(O, hd + s_max, num_q=4, num_kv=2, head_dim=hd, page_len=64, window=0,
+                  seqs=[(32 * s_max, 1), (40, 1), (0, 1)])
+    check(gpu, O, c, s_max)

@@ -30,6 +30,8 @@
 // split order with the reference's merge (corrections masked by l > 0, a
 // 16-lane tree per batch of 16 splits, the first contributing split
 // multiplied, the rest fma-accumulated).
+#include <algorithm>
+
 #include "bq_kernels.hpp"
 #include "bq_device.hpp"
 
@@ -80,13 +82,12 @@ __device__ inline float readlane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// workgroups of k_flash_attn_rows per group of 16 / G tokens: four tokens each
-// where it takes them one per wave
-__host__ __device__ constexpr int attn_rows_parts(int G) { return G <= 2 ? 4 / G : 1; }
-// whether it does so in blocks where no window slides
-__host__ __device__ constexpr bool attn_rows_lone(int G, int s_max) {
-  return G <= 2 && s_max > 1 && s_max < 16 / G;
-}
+// whether k_flash_attn_rows has blocks that it takes a wave per token (LONE)
+__host__ __device__ constexpr bool attn_rows_lone(int G, int s_max) { return G <= 2 && s_max > 1; }
+// and how long a split from position 0 has to be, at the end of a block, for
+// its groups to beat that (200 tokens from position 0, two splits: 21 against
+// 27 us; 70 tokens, four splits of up to 18: 14.7 / 14.2)
+constexpr int kRowsSplitLen = 48;
 
 // token metadata shared by the attention and merge kernels
 struct TokRange {
@@ -557,9 +558,13 @@ __device__ __forceinline__ void flash_attn_wave(const AttnArgs& a, int tok, int 
     // unchanged bit for bit (acc is never -0: it starts at +0 and only an
     // exact -0 product added to -0 gives -0), so the loop needs no branch.
     // The weights go through LDS, from G = 4 as [p][head % 4][head / 4]: lane
-    // L reads those of heads L % 4, + 4, ..., the MFMA's rows (a row of four
-    // fmaf in 2.3 cycles a lane against 2.6 to 4.2 for each v_fma); else as
-    // [p][head], read broadcast.
+    // L reads those of heads L % 4, + 4, ..., the rows of the f32 MFMA that
+    // takes four heads' fmaf at once; else as [p][head], read broadcast.  What
+    // the MFMA gives is fewer instructions in a wave's chain.  Head 512, eight
+    // heads, attention and merge: one sequence of 100 positions 15.8 us with
+    // v_fma, 14.7 so; 4 x 3000 29.1 / 27.9; 16 x 4096 55.0 / 53.9, where the
+    // SIMDs are full (the attention alone 36.4 / 37.5).  Sixteen heads, 8 x
+    // 3000: head 512 22.6 / 20.4 for the attention, head 64 10.0 / 9.1.
     if constexpr (G >= 4) {
 #pragma unroll
       for (int i = 0; i < NI; ++i)
@@ -671,15 +676,16 @@ __global__ __launch_bounds__(256, HD * G >= 8192 ? 1 : 2) void k_flash_attn(Attn
 // 400 vector instructions per wave.  The block of 2048 tokens from position 0
 // (sliding, head 256): 598 -> 412 us, attention alone 403 -> 222 us against a
 // wave per 8 tokens on v_fma; 700 + 411 tokens (full, head 512): 699 -> 396 us.
-// LONE: the instance of split plans whose blocks without a sliding window run
-// a wave per token; four waves per SIMD for those (200 tokens at position 500,
-// the block 140 -> 128 us), where the groups' own code wants the registers of
-// three (2048 tokens 330 us, with four 340).
+// LONE: the instance of split plans with one or two heads per kv head, whose
+// sets need several tokens to fill a group's rows: a workgroup with few takes
+// four tokens, a wave each, as k_flash_attn does.  A group walks its tiles in
+// the time of about three such waves, so it pays from three tokens per set.
 template <int HD, int G, bool LONE>
-__global__ __launch_bounds__(256, LONE ? 4 : HD >= 512 ? 2 : 3) void k_flash_attn_rows(AttnArgs a, int nblk) {
+__global__ __launch_bounds__(256, HD >= 512 ? 2 : 3) void k_flash_attn_rows(AttnArgs a, int nblk) {
   constexpr int C = HD / 64;    // 64-byte K chunks per row; column tiles per wave
   constexpr int TPW = 16 / G;   // tokens per group
   constexpr int NL = G >= 4 ? 1 : 4 / G;  // tokens among a lane's four rows
+  constexpr int NT = 16 * TPW;  // tokens per block
   // a step's weights [position][row]; corrections, weight sums (row 4: a spare)
   // and maxima [tile][row]
   __shared__ __attribute__((aligned(16))) float s_w[64 * 16];
@@ -707,51 +713,85 @@ __global__ __launch_bounds__(256, LONE ? 4 : HD >= 512 ? 2 : 3) void k_flash_att
   // (every other block's groups in reverse: a CU takes every 32nd workgroup of
   // its XCD, which would be the longest ranges of each block for some CUs and
   // the shortest for others)
-  const int cls = (item / 16 + part) & 1 ? 15 - item % 16 : item % 16;
-  const int t0 = (nblk - 1 - item / 16) * 16 * TPW;
+  const int cls = (item / 16) & 1 ? 15 - item % 16 : item % 16;
+  const int t0 = (nblk - 1 - item / 16) * NT, t1 = min(t0 + NT, a.T);
   const int run0 = run_of(a.runs, a.num_runs, t0);
   auto run_from = [&](int tok) {  // run_of(tok), tok >= t0
     int r = run0;
     while (r + 1 < a.num_runs && tok >= a.runs[r + 1].buf_start) ++r;
     return r;
   };
-  // groups take tokens 16 apart where some window of the block slides (equal
-  // starts mod 16), and neighbours where every range starts at position 0 (no
-  // tile of one is past the other)
-  int tok0 = t0 + cls * TPW, step = 1;
-  if (a.window > 0) {
-    bool slides = false;
+  // whether f(position) holds for a token of the block
+  auto any_pos = [&](auto f) {
+    bool x = false;
 #pragma unroll
-    for (int q = 0; q < 16 * TPW; q += kWave) {
+    for (int q = 0; q < NT; q += kWave) {
       const int tok = t0 + q + lane;
-      if (q + lane < 16 * TPW && tok < a.T) {
+      if (tok < t1) {
         const KvRun run = a.runs[run_from(tok)];
-        slides |= run.base_pos + (tok - run.buf_start) >= a.window;
+        x |= f(run.base_pos + (tok - run.buf_start));
       }
     }
-    if (__ballot(slides)) { tok0 = t0 + cls; step = 16; }
-  }
+    return __ballot(x) != 0;
+  };
+  // the first token's position and, in a block of one run, the last one's
+  const bool one = run0 + 1 >= a.num_runs || a.runs[run0 + 1].buf_start >= t1;
+  const int pos0 = a.runs[run0].base_pos + (t0 - a.runs[run0].buf_start), pos1 = pos0 + (t1 - 1 - t0);
+  // Groups take neighbours where every range starts at position 0 (no tile of
+  // one is past the other), and tokens 16 apart where windows slide (equal
+  // starts mod 16).
+  int tok0 = t0 + cls * TPW, step = 1;
+  // LONE, from position 0: split s starts at s * ceil(L / S), so with fewer
+  // splits than the group has tokens those that start together are S neighbours
+  // (from a position that S divides), and equal mod 16 those 16 S, 32 S, ...
+  // on.  sn > 0: the group is these, sn = S, counted round the block; S divides
+  // the group, so the block's end fits its beginning.
+  int sn = 0, turn = 0;
   if constexpr (LONE) {
-    // Where nothing slides, two neighbours' splits start together only if
-    // ceil(L / S) is the same for both: with fewer splits than tokens a group
-    // would be several small sets, and a wave per token is faster (200 tokens
-    // from position 0, two splits: the block 83 against 74 us)
-    if (step == 1) {
-      const int tok = tok0 + 4 * part + wave;
-      if (tok < a.T) flash_attn_wave<HD, G>(a, tok, kvh, s, s_w + wave * 16 * G);
+    // three tokens per group of those 16 (S) apart, or fewer at the end of a
+    // long chunk, whose other blocks fill the chip; the launch has the groups then
+    const bool spread = t1 - t0 >= 48 || nblk > 1;
+    bool lone = true;
+    if (a.window > 0 && pos0 >= a.window - 1) {  // every window of the block slides
+      lone = !(spread &&
+               (one || !any_pos([&](int pos) { return pos < a.window - 1; })));
+      tok0 = t0 + cls;
+      step = 16;
+    } else if (one && (a.window <= 0 || pos1 < a.window) && pos1 + 1 >= a.s_max * kRowsSplitLen &&
+               (a.s_max >= TPW || (TPW % a.s_max == 0 && spread))) {
+      lone = false;
+      if (a.s_max < TPW) {
+        sn = a.s_max;
+        turn = pos0 % sn;
+      }
+    }
+    if (lone) {
+      // the block's tokens from the last, over its workgroups of all parts
+      const int wgs = nblk > 1 ? NT / 4 : (a.T + 3) / 4;
+      const int tok = t0 + 4 * (wgs - 1 - (part * 16 + item % 16)) + wave;
+      if (part * 16 + item % 16 < wgs && tok < a.T)
+        flash_attn_wave<HD, G>(a, tok, kvh, s, s_w + wave * 16 * G);
       return;
     }
     if (part > 0) return;
+  } else if (a.window > 0 && (one ? pos1 >= a.window : any_pos([&](int pos) { return pos >= a.window; }))) {
+    tok0 = t0 + cls;
+    step = 16;
   }
-  if (tok0 >= a.T) return;
+  // token k of the group (none from a.T on)
+  auto token = [&](int k) {
+    if (!LONE || sn == 0) return tok0 + step * k;
+    return t0 + ((k % sn + sn * cls + 16 * sn * (k / sn) - turn) & (NT - 1));
+  };
+  if (sn == 0 && tok0 >= a.T) return;
   const int64_t kvs = (int64_t)a.num_kv * HD;
 
   // token lane % TPW of the group: its positions [t_beg, t_end) of this split,
   // its number of splits (0: no token), its set
   int t_beg = 0, t_end = 0, t_S, t_set = -1, nsets = 0, tiles = 0;
   {
-    const int tok = tok0 + step * (lane % TPW);
-    const int r = run_from(tok);
+    const int tok = token(lane % TPW);
+    const int r = run_from(min(tok, a.T - 1));
     const KvRun run = a.runs[r];
     const int pos = run.base_pos + (tok - run.buf_start);
     const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
@@ -792,7 +832,7 @@ __global__ __launch_bounds__(256, LONE ? 4 : HD >= 512 ? 2 : 3) void k_flash_att
   // 4 g + i, position p.
   const v4i zero4 = {0, 0, 0, 0};
   {
-    const int tok = min(tok0 + step * (p16 / G), a.T - 1);  // (rows without a token: never used)
+    const int tok = min(token(p16 / G), a.T - 1);  // (rows without a token: never used)
     const int64_t qrow = (int64_t)tok * a.num_q + kvh * G + p16 % G;
     int part = 0;
 #pragma unroll
@@ -972,7 +1012,7 @@ __global__ __launch_bounds__(256, LONE ? 4 : HD >= 512 ? 2 : 3) void k_flash_att
   // (acc * c) * (1/(l * c)) with c = fast_exp(0)); other splits are partials
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int r = 4 * grp + i, k = r / G, tok = tok0 + step * k;
+    const int r = 4 * grp + i, k = r / G, tok = token(k);
     const float lr = __shfl(l, r, kWave), mr = __shfl(m, r, kWave);
     const int S = __shfl(t_S, k, kWave);
     if (s >= S) continue;  // no such token, or no such split of it
@@ -1117,7 +1157,11 @@ static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
   const int tpw = 16 / gqa, nblk = (a.T + 16 * tpw - 1) / (16 * tpw);
   if (a.s_max == 1 || a.T >= 2 * tpw * a.num_runs) {
     const bool lone = attn_rows_lone(gqa, a.s_max);
-    const dim3 g(nblk * 16 * (lone ? attn_rows_parts(gqa) : 1) * a.num_kv * a.s_max);
+    // LONE: workgroups for four tokens each, and for a block's 16 groups where
+    // it can have them
+    const int need = (a.T + 3) / 4, groups = a.T < 48 ? need : std::max(16, need);
+    const int per = !lone ? nblk * 16 : nblk > 1 ? nblk * 4 * tpw : groups;
+    const dim3 g(per * a.num_kv * a.s_max);
     switch (gqa) {
       case 1:
         if (lone) hipLaunchKernelGGL((k_flash_attn_rows<HD, 1, true>), g, b, 0, st, a, nblk);

@@ -251,3 +251,41 @@ def test_attention_merge_instances(gpu, O, hd, s_max):
     c = make_case(O, hd + s_max, num_q=4, num_kv=2, head_dim=hd, page_len=64, window=0,
                   seqs=[(32 * s_max, 1), (40, 1), (0, 1)])
     check(gpu, O, c, s_max)
+
+
+@pytest.mark.parametrize("gqa,s_max,window,seqs", [
+    # blocks of 128 tokens (two heads per kv head)
+    (2, 2, 0, [(0, 150)]),            # neighbours in pairs, a last block of 22
+    (2, 2, 0, [(101, 130)]),          # ... counted round the block from an odd position
+    (2, 4, 0, [(243, 77)]),           # fours, one short block
+    (2, 3, 0, [(200, 140)]),          # three splits do not divide the group: a wave per token
+    (2, 2, 0, [(0, 70), (5, 80)]),    # a block of two runs: a wave per token
+    (2, 8, 0, [(400, 30)]),           # neighbours in launches of fewer than 16 groups
+    (2, 9, 0, [(500, 60)]),
+    (2, 2, 64, [(0, 300)]),           # windows slide in the later blocks only
+    (2, 3, 50, [(49, 49)]),           # all slide: 49 tokens in groups,
+    (2, 3, 50, [(49, 47)]),           # 47 a wave each
+    (2, 2, 40, [(100, 70), (60, 90)]),
+    (2, 2, 40, [(100, 70), (0, 90)]),
+    # blocks of 256 tokens (a head per kv head)
+    (1, 2, 0, [(30, 300)]),
+    (1, 4, 0, [(333, 90)]),
+    (1, 8, 0, [(700, 60)]),
+    (1, 5, 0, [(0, 71)]),
+    (1, 3, 64, [(0, 280)]),
+])
+def test_attention_row_group_forms(gpu, O, gqa, s_max, window, seqs):
+    # every form of a split plan's groups, over several blocks and kv heads
+    c = make_case(O, gqa + 10 * s_max + window, num_q=2 * gqa, num_kv=2, head_dim=64, page_len=64,
+                  window=window, ring_pages=4, seqs=seqs)
+    check(gpu, O, c, s_max)
+
+
+@pytest.mark.parametrize("s_max", [1, 2])
+@pytest.mark.parametrize("gqa", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("hd", [64, 128, 256, 512])
+def test_attention_row_group_instances(gpu, O, hd, gqa, s_max):
+    # a chunk in every instance: groups in its first run, some in the second
+    c = make_case(O, hd + gqa + s_max, num_q=gqa, num_kv=1, head_dim=hd, page_len=64,
+                  window=0 if gqa & 5 else 90, ring_pages=4, seqs=[(101, 131), (3, 20)])
+    check(gpu, O, c, s_max)

@@ -45,7 +45,7 @@ def kernels(tmp_path_factory):
             for d, v in zip(names, found.values())}
 
 
-@pytest.mark.parametrize("kernel,instances", [("k_flash_attn", 20)])
+@pytest.mark.parametrize("kernel,instances", [("k_flash_attn", 20), ("k_flash_attn_rows", 28)])
 def test_no_scratch(kernels, kernel, instances):
     mine = {n: v for n, v in kernels.items() if n.startswith(kernel + "<")}
     assert len(mine) == instances, sorted(mine)

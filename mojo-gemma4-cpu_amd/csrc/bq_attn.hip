@@ -1150,12 +1150,21 @@ hipError_t launch_attn_prep(const PrepArgs& args, int head_dim, hipStream_t st) 
 template <int HD>
 static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
   const dim3 b(256);
-  // Row groups need neighbours in a run to share tiles with: one-split plans
-  // (many tokens), and split plans with two groups' tokens per run (200 tokens
-  // of one run at position 2000, sliding: 178 -> 102 us).  A decode step's
-  // tokens share nothing: a wave each.
+  // Row groups need neighbours in a run to share tiles with: two groups' tokens
+  // per run, and 20 with four heads or fewer, whose sliding windows share tiles
+  // 16 tokens apart (200 tokens of one run at position 2000, sliding, both
+  // kernels: a wave per token 130 us, groups 54; 16 tokens of four heads 14.6 /
+  // 23).  A decode step's tokens share nothing and take a wave each (one split,
+  // two heads of 256, 512 sequences of 1000 positions 325 us, in groups 496;
+  // eight of 512, 256 sequences of 1500 545 / 700).  One-split plans of 16
+  // heads, which fill a group's rows by themselves, and of eight up to head 256
+  // stay in groups, whose four waves walk a range in a quarter of the steps (16
+  // heads of 256, 600 sequences of 1500 346 / 176; eight of 128, 512 sequences
+  // 221 / 165).
   const int tpw = 16 / gqa, nblk = (a.T + 16 * tpw - 1) / (16 * tpw);
-  if (a.s_max == 1 || a.T >= 2 * tpw * a.num_runs) {
+  const int chunk = gqa >= 8 ? 2 * tpw : std::max(2 * tpw, 20);
+  if (a.T >= chunk * a.num_runs ||
+      (a.s_max == 1 && (gqa == 16 || (gqa == 8 && HD <= 256)))) {
     const bool lone = attn_rows_lone(gqa, a.s_max);
     // LONE: workgroups for four tokens each, and for a block's 16 groups where
     // it can have them

@@ -289,3 +289,12 @@ def test_attention_row_group_instances(gpu, O, hd, gqa, s_max):
     c = make_case(O, hd + gqa + s_max, num_q=gqa, num_kv=1, head_dim=hd, page_len=64,
                   window=0 if gqa & 5 else 90, ring_pages=4, seqs=[(101, 131), (3, 20)])
     check(gpu, O, c, s_max)
+
+
+@pytest.mark.parametrize("gqa,hd", [(1, 64), (2, 256), (4, 128), (8, 256), (8, 512), (16, 64)])
+@pytest.mark.parametrize("window", [0, 40])
+def test_attention_one_split_decode(gpu, O, gqa, hd, window):
+    # one-split plans of many sequences of one token, and of chunks beside them
+    c = make_case(O, gqa + hd + window, num_q=2 * gqa, num_kv=2, head_dim=hd, page_len=64,
+                  window=window, ring_pages=4, seqs=[(37 * i % 150, 1 + 2 * (i % 9 == 0)) for i in range(40)])
+    check(gpu, O, c, 1)

@@ -1163,13 +1163,16 @@ static hipError_t launch_attn_hd(const AttnArgs& a, int gqa, hipStream_t st) {
   // 221 / 165).
   const int tpw = 16 / gqa, nblk = (a.T + 16 * tpw - 1) / (16 * tpw);
   const int chunk = gqa >= 8 ? 2 * tpw : std::max(2 * tpw, 20);
-  if (a.T >= chunk * a.num_runs ||
-      (a.s_max == 1 && (gqa == 16 || (gqa == 8 && HD <= 256)))) {
-    const bool lone = attn_rows_lone(gqa, a.s_max);
-    // LONE: workgroups for four tokens each, and for a block's 16 groups where
-    // it can have them
-    const int need = (a.T + 3) / 4, groups = a.T < 48 ? need : std::max(16, need);
-    const int per = !lone ? nblk * 16 : nblk > 1 ? nblk * 4 * tpw : groups;
+  // LONE: workgroups for four tokens each, and for a block's 16 groups where it
+  // can have them
+  const bool lone = attn_rows_lone(gqa, a.s_max);
+  const int need = (a.T + 3) / 4, groups = a.T < 48 ? need : std::max(16, need);
+  const int per = !lone ? nblk * 16 : nblk > 1 ? nblk * 4 * tpw : groups;
+  // (a launch has fewer than 2^24 workgroups of 256: past that a wave per token,
+  // of which a workgroup has four)
+  const bool fits = (int64_t)per * a.num_kv * a.s_max < (1 << 24);
+  if (fits && (a.T >= chunk * a.num_runs ||
+               (a.s_max == 1 && (gqa == 16 || (gqa == 8 && HD <= 256))))) {
     const dim3 g(per * a.num_kv * a.s_max);
     switch (gqa) {
       case 1:

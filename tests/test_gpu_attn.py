@@ -298,3 +298,32 @@ def test_attention_one_split_decode(gpu, O, gqa, hd, window):
     c = make_case(O, gqa + hd + window, num_q=2 * gqa, num_kv=2, head_dim=hd, page_len=64,
                   window=window, ring_pages=4, seqs=[(37 * i % 150, 1 + 2 * (i % 9 == 0)) for i in range(40)])
     check(gpu, O, c, 1)
+
+
+def test_attention_more_groups_than_a_launch(gpu, O):
+    # 2^24 row groups of one token: a launch takes fewer, so it is a wave per
+    # token; the first and the last tokens as in calls of their own
+    import torch
+    hd, nq, nkv, page, T = 64, 256, 16, 1024, 1 << 20
+    d = "cuda"
+    g = torch.Generator(device=d).manual_seed(5)
+    i8 = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device=d, generator=g)  # noqa: E731
+    q, kc, vc = i8(T, nq * hd), i8(2 * page, nkv * hd), i8(2 * page, nkv * hd)
+    ks, vs = torch.rand(2 * page, nkv, device=d) + 1, torch.rand(2 * page, nkv, device=d) + 1
+    qb = torch.zeros(T, nq, device=d)
+    fq = torch.full((T, nq), 0.01, device=d)
+    rows = torch.tensor([0, page], dtype=torch.int32, device=d)
+
+    def call(t0, n):
+        runs = torch.tensor([[0, t0, 0, 2]], dtype=torch.int32, device=d)
+        s = slice(t0, t0 + n)
+        return gpu.attention(q[s], qb[s], fq[s], kc, ks, vc, vs, runs, rows, nq, nkv, hd, 3, 10,
+                             page - 1, 1, s_max=1)[0]
+
+    print(f"attention T={T} nq={nq} nkv={nkv} hd={hd}", flush=True)
+    out = call(0, T)
+    torch.cuda.synchronize()
+    same = [torch.equal(out[t0:t0 + 100], call(t0, 100)) for t0 in (0, T // 2 - 7, T - 100)]
+    del q, qb, fq, out
+    torch.cuda.empty_cache()  # (120 GB, most of it workspace)
+    assert same == [True, True, True]

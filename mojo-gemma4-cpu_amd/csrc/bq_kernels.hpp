@@ -109,7 +109,7 @@ hipError_t launch_moe_down_tiled(const int8_t* b_i8, const float* b_sa, const in
                                  const Route* routes, const int8_t* w_d, const float* d_scale,
                                  float* y, int experts, int max_routes, int hidden, int inter,
                                  int block, int bm, hipStream_t st);
-int moe_tile_bm(int max_routes, int experts);
+int moe_tile_bm(int max_routes, int experts, bool dense);
 
 // kernels/flash_sample.mojo:21-28 SamplingParams and :120-134
 // SampleOutcome[256], laid out as the Mojo structs are (bq_api.h mirrors them)

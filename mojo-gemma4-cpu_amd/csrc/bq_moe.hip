@@ -18,6 +18,8 @@
 #include "bq_kernels.hpp"
 #include "bq_sched.hpp"
 
+#include <cmath>
+
 namespace bq {
 
 // One workgroup per expert e.  The (expert, token, k) order puts route slot
@@ -614,16 +616,26 @@ static inline int mtile_bound(int max_routes, int experts, int bm) {
 // tiled tiles once each expert's weights can be reused.  The tile is sized
 // so that nearly every expert fits in one m-tile (mean + 4 standard
 // deviations of a binomial count): then each expert's weights stream from
-// HBM once instead of once per m-tile.  From 15 routes per expert most experts
-// would fill two 16-row tiles and stream their weights twice (top-8 of 128,
-// the expert block in 16 / 64-row tiles: 200 tokens 168 / 172 us, 256 tokens
-// 209 / 174, 333 tokens 254 / 181; 100 tokens of 64 experts 95 / 97, 160 138 /
-// 103; with the dense MLP 200 tokens 224 / 244, 256 286 / 264).
-int moe_tile_bm(int max_routes, int experts) {
+// HBM once instead of once per m-tile.
+// Between 15 and 24 routes per expert the 16-row tiles read the weights of an
+// expert with more than 16 records twice; the tiled kernels take about as long
+// for few experts as for many.  They pay from about 13 such experts (hidden
+// 2816, inter 704, the expert block in 16 / 64-row tiles: 128 experts, 15
+// routes each, 201 / 178 us; 64, 15 110 / 101; 32, 17 75 / 68, 15 64 / 69; 16,
+// 17 50 / 52; 8, 19 38 / 49), and from 40 with the dense MLP, whose own rows
+// then take a launch of 64-token workgroups (128, 15 247 / 234; 96, 17 220 /
+// 205, 15 198 / 204; 64, 19 164 / 156, 17 151 / 155; 32, 23 119 / 123; 16, 21
+// 74 / 96; 4, 15 41 / 77).
+int moe_tile_bm(int max_routes, int experts, bool dense) {
   if (tune().moe_bm) return tune().moe_bm;
-  const int per = max_routes / (experts > 0 ? experts : 1);
-  if (per < 15) return 16;
-  const double hi = per + 4.0 * __builtin_sqrt((double)per);
+  const double per = (double)max_routes / (experts > 0 ? experts : 1);
+  if (per < 15.0) return 16;
+  if (per < 24.0) {
+    // experts with more than 16 records: a Poisson count's tail as a normal one's
+    const double twice = experts * 0.5 * erfc((16.5 - per) / __builtin_sqrt(2.0 * per));
+    if (twice < (dense ? 40.0 : 13.0)) return 16;
+  }
+  const double hi = per + 4.0 * __builtin_sqrt(per);
   if (hi > 192.0) return 256;
   if (hi > 128.0) return 192;  // 2048 tokens x top-8 / 128 experts: 128 + 45
   if (hi > 64.0) return 128;
@@ -649,7 +661,7 @@ hipError_t launch_moe_phase1(const int8_t* x_i8, const float* x_sa, const int32_
   }
   const int moe_rows = max_routes > 0 ? mtile_bound(max_routes, experts, 16) : 0;
   if (max_routes > 0) {
-    const int bm = moe_tile_bm(max_routes, experts);
+    const int bm = moe_tile_bm(max_routes, experts, has_dense);
     if (bm >= 64 && inter % 64 == 0) {
       const hipError_t r = launch_moe_gate_up_tiled(x_i8, x_sa, eo, routes, w_gu, gu_scale, bucket,
                                                     bi8, bsa, experts, max_routes, hidden, inter,
@@ -723,7 +735,7 @@ hipError_t launch_moe_phase2(const int8_t* bucket_i8, const float* bucket_sa, co
   };
   bool dense_done = !has_dense;
   if (max_routes > 0) {
-    const int bm = moe_tile_bm(max_routes, experts);
+    const int bm = moe_tile_bm(max_routes, experts, has_dense);
     if (bm >= 64 && hidden % 128 == 0) {
       // see launch_moe_down_tiled; BQ_MOE_BM_DOWN overrides the down tile alone
       const int bm_down = tune().moe_bm_down ? tune().moe_bm_down : tune().moe_bm ? bm : 64;

@@ -310,3 +310,12 @@ def test_attention_waves_switch(gpu, O, tune_env, waves, name):
     w = SHAPES[name].get("window", 0)
     s_max = gpu.attention_splits(c.T, c.num_kv, w if w else int(c.positions.max()) + 1)
     check(gpu, O, c, s_max)
+
+
+@pytest.mark.parametrize("T,E,k", [(30, 4, 2), (47, 4, 2), (48, 4, 2), (60, 16, 4), (90, 16, 4), (120, 32, 4),
+                                   (150, 32, 4), (120, 64, 8), (140, 64, 8), (150, 64, 8)])
+def test_moe_tile_line(gpu, O, T, E, k):
+    # 12 to 24 routes per expert, both sides of the line between the 16-row and
+    # the tiled kernels, which lies elsewhere with the dense MLP
+    _moe_check(gpu, O, T, E, k)
+    _ffn_check(gpu, O, T, E, k)

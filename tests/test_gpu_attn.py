@@ -83,8 +83,8 @@ def test_attention_many_splits(gpu, O):
 
 
 def test_attention_splits_beyond_one_stage(gpu, O):
-    # 282 splits for the long token: the many-split merge stages them in two
-    # LDS passes (240 + 42)
+    # 282 splits for the long token: the merge takes them 64 corrections and 32
+    # rows at a time, the last batch of each short
     c = make_case(O, 12, num_q=2, num_kv=1, head_dim=64, page_len=64, window=0,
                   seqs=[(9000, 1), (100, 1)])
     check(gpu, O, c, 300)
@@ -98,7 +98,7 @@ def test_attention_splits_beyond_one_stage(gpu, O):
 ])
 def test_attention_single_split_groups(gpu, O, gqa, hd, window, seqs):
     # one split per token (s_max = 1): tokens t, t + 16, ... of a run share a
-    # wave when their tile grids coincide; the rest run one per pass
+    # group; those whose tile grids coincide are one set of its tiles
     c = make_case(O, gqa * 3 + hd + window, num_q=2 * gqa, num_kv=2, head_dim=hd, page_len=64,
                   window=window, ring_pages=4, seqs=seqs)
     check(gpu, O, c, 1)

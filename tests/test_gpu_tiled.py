@@ -21,11 +21,12 @@ def test_dense_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B):
     tune_env(BQ_TILE_BM=bm, BQ_TILE_BN=bn, BQ_MF=mf)
     N = 384  # 1.5 n-tiles at bn=256; N=2816 tails are covered in test_gpu_parity
     wf = O.bf16_to_f32(O.synth_normal_bf16(3, 0.02, (N, K)))
-    q, s = O.rotate_and_quant(wf, B or 128)
+    wide = 128 if K % 128 == 0 else 64
+    q, s = O.rotate_and_quant(wf, B or wide)
     W = gpu.ButterquantWeight(gpu.retile(dev(q.reshape(-1)), N, K), dev(s), N, K)
     x = O.synth_normal_bf16(4, 1.0, (M, K))
     if B is None:
-        xq, sa = O.norm_quant(x, np.full(K, ONE, np.uint16), 128 if K % 128 == 0 else 64)
+        xq, sa = O.norm_quant(x, np.full(K, ONE, np.uint16), wide)
         ob, of = gpu.linear(dev(xq), dev(sa), W, want_f32=True)
         p, cs = O.pack_and_colsum(q)
         rb, rf = O.linear(xq, sa, p, s, cs, N)
@@ -38,12 +39,57 @@ def test_dense_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B):
     np.testing.assert_array_equal(host(ob), rb)
 
 
+@pytest.mark.parametrize("mf", [16, 32])
 @pytest.mark.parametrize("bm,bn", [(192, 128), (192, 256), (256, 256)])
-@pytest.mark.parametrize("M,K,B", [(193, 640, None), (511, 384, None), (255, 1024, 256), (400, 2112, 64)])
-def test_dense_tall_tiles(gpu, O, tune_env, bm, bn, M, K, B):
+@pytest.mark.parametrize("M,K,B", [(193, 704, None), (511, 320, None), (193, 640, None), (511, 384, None),
+                                   (255, 1024, 256), (400, 2112, 64)])
+def test_dense_tall_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B):
     # the taller tiles of large chunks: a last tile of one row, of all but one,
-    # odd k-steps, and 1.5 n-tiles
-    test_dense_tiles(gpu, O, tune_env, bm, bn, 16, M, K, B)
+    # 11 and 5 k-steps beside even counts (per-block tiles of these heights are
+    # 128 columns wide whatever bn), and 1.5 n-tiles
+    test_dense_tiles(gpu, O, tune_env, bm, bn, mf, M, K, B)
+
+
+@pytest.mark.parametrize("M,ns,K,B", [
+    (17, (8224,), 320, None),                   # 32 x 128
+    (32, (8224,), 704, None),
+    (200, (2784, 544, 544), 320, None),          # 64 x 128
+    (300, (4000, 2016, 2016), 704, None),       # 128 x 128
+    (511, (4128, 2080, 2080), 320, None),       # 192 x 128
+    (700, (8224, 1056), 704, None),             # 128 x 256
+    (1111, (8224, 1056), 320, None),            # 192 x 256
+    (2047, (4000, 1952, 1952), 320, None),      # 256 x 256
+    (129, (2784,), 704, 64),                    # per-block 64 x 128
+    (1000, (5600,), 704, 64),                   # per-block 128 x 256
+    (2047, (2848,), 704, 64),                   # per-block 192 x 128
+])
+def test_picked_tiles(gpu, O, M, ns, K, B):
+    """The tile that the launcher picks on 256 CUs, by itself, with segments of
+    no whole tiles: against the calls of 16 rows and one weight (k_linear_skinny,
+    no tiles), whose last rows are compared with the oracle, bit-exact."""
+    import torch
+    qs = [O.rotate_and_quant(O.bf16_to_f32(O.synth_normal_bf16(3 + i, 0.02, (n, K))), 64)
+          for i, n in enumerate(ns)]
+    Ws = [gpu.ButterquantWeight(gpu.retile(dev(q.reshape(-1)), n, K), dev(s), n, K)
+          for (q, s), n in zip(qs, ns)]
+    x = O.synth_normal_bf16(4, 1.0, (M, K))
+    xq, sa = O.norm_quant(x, np.full(K, ONE, np.uint16), 64) if B is None else O.block_quant(x, B, True)
+    dx, ds = dev(xq), dev(sa)
+    one = (lambda a, b, W: gpu.linear(a, b, W)) if B is None else \
+        (lambda a, b, W: gpu.block_linear(a, b, W, B))
+    outs = (one(dx, ds, Ws[0]),) if len(ns) == 1 else \
+        gpu.linear_pair(dx, ds, *Ws) if len(ns) == 2 else gpu.qkv(dx, ds, *Ws)
+    r0 = (M - 1) // 16 * 16
+    for out, W, (q, s) in zip(outs, Ws, qs):
+        rows = torch.cat([one(dx[r:r + 16], ds[r:r + 16], W) for r in range(0, M, 16)])
+        assert torch.equal(out, rows)
+        if B is None:
+            p, cs = O.pack_and_colsum(q)
+            ref, _ = O.linear(xq[r0:], sa[r0:], p, s, cs, W.n_rows)
+        else:
+            p, cs = O.pack_and_colsum(q, B, False)
+            ref, _ = O.block_linear(xq[r0:], sa[r0:], p, s, cs, W.n_rows, B)
+        np.testing.assert_array_equal(host(out[r0:]), ref)
 
 
 @pytest.mark.parametrize("mf", [16, 32])

@@ -430,7 +430,8 @@ void k_gemv_m1_1(BQ_SEG1_PARAMS) {
 // of 128 x 128 58, one of 192 x 256 39; 512 x 4096 at K = 4096 one of 64 x 128
 // 14, 128 x 256 36.  Per-block: 2048 x 2816 at K = 4096 two rounds of 128 x
 // 128 74, one of 192 x 128 50; 1111 x 2816 at K = 8192 396 of 64 x 128, two to
-// a CU, 75, 198 of 128 x 128 66).
+// a CU, 75, 198 of 128 x 128 66).  Every tile's two-stage ring fits LDS beside
+// the scales of 64 K blocks, the most a call has.
 static void pick_linear_tile(const LinArgs& a, int per_block, int& bm, int& bn) {
   struct Tile { int bm, bn; float cost; };
   static const Tile row[] = {{64, 128, 3.5f}, {128, 128, 6.5f}, {192, 128, 9.6f},
@@ -447,8 +448,7 @@ static void pick_linear_tile(const LinArgs& a, int per_block, int& bm, int& bn) 
     // (64 x 128 per-block tiles run two to a CU, at 9.1 the pair)
     if (per_block && t[i].bm == 64 && rounds > 1.0f)
       rounds = (float)((tiles + 2 * tune().cus - 1) / (2 * tune().cus)) * (9.1f / 5.5f);
-    if (i > 0 && (rounds * t[i].cost >= best || !linear_tile_fits(a, per_block, t[i].bm, t[i].bn)))
-      continue;
+    if (i > 0 && rounds * t[i].cost >= best) continue;
     best = rounds * t[i].cost;
     bm = t[i].bm;
     bn = t[i].bn;
@@ -459,8 +459,8 @@ hipError_t launch_linear(const LinArgs& a, int per_block, hipStream_t st) {
   if (a.M <= 0) return hipSuccess;
   // Past 16 rows the tiled kernels take over once they have workgroups enough:
   // a few dozen rows over few columns leave most CUs idle there, where 16 x 16
-  // tiles with K split over 16 waves fill the chip, the weights read again from
-  // L2 for each 16 rows.  Per-row up to three such tiles per CU (with its
+  // tiles with K split over 16 waves fill the chip, though the weights are read
+  // again for each 16 rows.  Per-row up to three such tiles per CU (with its
   // norm-quant, 32 x 4096 at K 4096 25.9 -> 20.4 us, 64 x 1024 19.4 -> 14.0, but
   // 48 x 8192 at K 2816 6 us longer), per-block up to six (32 x 2816 at K 8192
   // 31 -> 12 us, 128 rows 1.3 us shorter).  (A switch of the tiled kernels

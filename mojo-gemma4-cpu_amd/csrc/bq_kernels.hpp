@@ -99,8 +99,6 @@ hipError_t launch_norm_linear(const LinArgs& a, const NormArgs& nq, hipStream_t 
 struct Route { int32_t token; float weight; };
 
 hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, int bn, hipStream_t st);
-// whether a bm x bn tile's operand ring and block scales fit in LDS
-bool linear_tile_fits(const LinArgs& a, int per_block, int bm, int bn);
 hipError_t launch_moe_gate_up_tiled(const int8_t* x_i8, const float* x_sa, const int32_t* eo,
                                     const Route* routes, const int8_t* w_gu, const float* gu_scale,
                                     uint16_t* bucket, int8_t* bi8, float* bsa, int experts,

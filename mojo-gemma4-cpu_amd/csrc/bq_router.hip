@@ -33,7 +33,11 @@ constexpr float kRouterSentinel = -1.0e30f;
 // It is memory latency: steps are loaded U at a time, one batch ahead of the
 // chains and the first ahead of the sums of squares (the feed-forward block
 // against a load round trip per step: 1 token 50.6 -> 47.9 us, 16 tokens 110.7
-// -> 103.5, 333 tokens 273 -> 252).
+// -> 103.5, 333 tokens 273 -> 252).  U is what the registers hold beside the
+// tile's sums: 11 for 2 x 4 tiles, which hidden 2816 (22 steps) ends in two
+// batches; fewer steps repeat their last one (these logits alone, 16
+// tokens, operands not in L2: hidden 512 4.6 -> 3.9 us, 1024 7.1 -> 4.5, 2816
+// 13.9 -> 6.5, 4096 17.8 -> 9.0).
 template <int TT, int EE, int CPL, int U>
 __global__ __launch_bounds__(256) void k_router_logits(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ proj,

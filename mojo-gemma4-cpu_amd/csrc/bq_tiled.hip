@@ -904,11 +904,6 @@ static void launch_bm(int bm, int bn, int nbuf, dim3 g, size_t dyn, hipStream_t 
 
 static inline int tile_bn(int bn) { return bn >= 256 ? 256 : 128; }
 
-bool linear_tile_fits(const LinArgs& a, int per_block, int bm, int bn) {
-  const size_t dyn = per_block ? (size_t)bm * (a.K / a.block) * sizeof(float) : 0;
-  return 2 * (size_t)(bm + bn) * 128 + dyn <= kLdsBytes;
-}
-
 hipError_t launch_linear_tiled(const LinArgs& a, int per_block, int bm, int bn, hipStream_t st) {
   const int bmv = bm >= 256 ? 256 : bm >= 192 ? 192 : bm >= 128 ? 128 : bm >= 64 ? 64 : 32;
   // (per-block tiles of 192 or 256 rows are 128 columns wide: launch_bm_mf)
